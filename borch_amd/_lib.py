@@ -94,6 +94,8 @@ SIGNATURES = {
                                    _c_i64, _c_p, _c_p, _c_p, _c_int, _c_p, _c_p, _c_p]),
     "bq_gemv_w8a32": (_c_int, [_c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_int, _c_p, _c_p]),
     "bq_linear_w8a32": (_c_int, [_c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_int, _c_p, _c_p]),
+    "bq_linear_w8a32_ws": (_c_int, [_c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_int, _c_p, _c_p,
+                                    _c_size, _c_p]),
     "bq_dequant_i8": (_c_int, [_c_p, _c_i64, _c_i64, _c_p, _c_p, _c_p]),
     "bq_attention_f32": (_c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p]),
     "bq_avgpool_linear_f32": (_c_int, [_c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_i64, _c_p, _c_p]),

@@ -4,15 +4,21 @@
 // kernels.ts:2695-2708) for streamed/windowed weights, and its `dequantInt8` unpack pass
 // (kernels.ts:1264-1274).
 //
-// gemv_w8a32_kernel (M <= 4, the decode shape; gemv_w8a32_mfma_kernel below for M = 5..8):
+// gemv_w8a32_kernel (M <= 4, the decode shape; the MFMA kernels below take more rows):
 // HBM-bound on the int8 weight — a quarter of the f32 bytes. Each wave owns RPW weight rows; a row is read as contiguous 1 KB
 // wave-loads (64 lanes x 16 bytes) and every load of the wave's rows is issued before any
 // arithmetic; each lane multiplies its 16 weights against the matching 16 activations
 // (L1/L2-resident, reused across the wave's rows) and the wave reduces the lane sums.
+#include <algorithm>
+
+#include "bq_bf16x3.h"
 #include "bq_common.h"
 
 namespace bq {
 
+// bq_gemm_ws_bytes(): 1024 tile counters, zero between launches, then the partial sums.
+constexpr size_t W8_CNT_BYTES = 4096;
+constexpr size_t W8_WS_BYTES = W8_CNT_BYTES + (size_t)416 * 4096 * 4;
 constexpr uint32_t W_OOB = 0x80000000u;
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t w_rsrc(const void* base, uint32_t bytes) {
@@ -20,11 +26,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t w_rsrc(const void* base, uint3
 }
 
 constexpr int WA_WAVES = 8;
-constexpr int WA_MMAX = 16;  // activation rows the GEMV kernels take (the MFMA one: 5..16)
-// From this many activation rows the MFMA kernel runs (4096 x 4096, us, per-wave / MFMA:
-// M=2 7.9 / 11.4, M=4 10.5 / 11.7, M=5 13.0 / 11.7, M=6 14.4 / 11.9, M=8 17.3 / 12.8).
-constexpr int WA_MFMA_MIN_M = 5;
-constexpr int WA_MPW = WA_MFMA_MIN_M - 1;  // activation rows the per-wave kernel takes
+constexpr int WA_MMAX = 16;  // activation rows bq_gemv_w8a32 takes
+constexpr int WA_MPW = 4;    // activation rows the per-wave kernel takes (4096 x 4096, M = 2 / 4: 7.9 / 10.5 us)
 constexpr int WA_XLDS = 16384;       // f32 activations staged through registers (64 KB of LDS)
 constexpr int WA_XLDS_BIG = 32768;   // staged by a load loop after the weights (128 KB of LDS)
 
@@ -191,7 +194,7 @@ __global__ __launch_bounds__(WA_WAVES * 64) void gemv_w8a32_kernel(const float* 
   }
 }
 
-// gemv_w8a32_mfma_kernel (2 <= M <= 8): the products on v_mfma_f32_16x16x4_f32. A
+// gemv_w8a32_mfma_kernel (5 <= M <= 16, short K): the products on v_mfma_f32_16x16x4_f32. A
 // workgroup owns 16 weight rows; its waves split K into 64-byte chunks (wave w takes
 // chunks w, w + 8, ...). Lane l holds 16 bytes of weight row l % 16 at K offset
 // 64 c + 16 (l / 16) and the 16 matching floats of activation row l % 16 (zero for rows
@@ -201,7 +204,6 @@ __global__ __launch_bounds__(WA_WAVES * 64) void gemv_w8a32_kernel(const float* 
 // order, within the same f32-accumulation bound. The per-wave kernel above reads every
 // activation row in every wave and does M FMAs a weight on the VALU: at M = 8, 17.3 us for
 // a 4096 x 4096 weight. Partial 16 x 16 blocks meet through LDS in wave order.
-typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int WM_ROWS = 16;
 template <int CPW>  // 64-byte chunks a wave: K <= CPW * 8 * 64
 __global__ __launch_bounds__(WA_WAVES * 64) void gemv_w8a32_mfma_kernel(const float* __restrict__ x, const int8_t* W,
@@ -280,70 +282,25 @@ __global__ __launch_bounds__(WA_WAVES * 64) void gemv_w8a32_mfma_kernel(const fl
   }
 }
 
-// ------------------------------------------------------------ W8A32 for any M: tiled
+// ------------------------------------------------- W8A32 above the decode rows: bf16 MFMA
 //
-// w8a32_gemm_kernel: out[m, n] = act(fl(fl(acc[m, n] * s[n]) + bias[n]) + res[m, n]) with
-// acc[m, n] = sum_k x[m, k] * q[n, k] accumulated in f32. The bf16 MFMA runs 16 times the
-// f32 MFMA rate on this chip, and every product fits it exactly:
-//  * q (|q| <= 127: 7 bits) is exact in bf16 (8 significant bits);
-//  * x is split into x = x1 + x2 + x3 with x1 the bf16 nearest x and x2 the bf16 nearest
-//    x - x1. x - x1 is a multiple of ulp_f32(x) below 2^-8 |x| (at most 16 significant
-//    bits), (x - x1) - x2 a multiple of it below 2^-16 |x| (at most 8), so x3 = (x - x1) - x2
-//    is exact in bf16 and the split loses nothing (|x| >= 2^-100, so no piece is subnormal).
-// Each x * q is then three exact products x_i * q (at most 15 significant bits), which three
-// v_mfma_f32_16x16x32_bf16 add into one f32 accumulator: the accumulation is the only
-// rounding before the per-channel scale, applied once to the sum. The reference's order
-// (the effective weight f32(q) * s rounded per element, then f32 FMAs, kernels.ts:2695-2708)
-// and this one are both within the f32-accumulation bound (K + 2) 2^-24 sum |x * w| of the
-// exact result on the effective weights.
+// out[m, n] = act(fl(fl(acc[m, n] * s[n]) + bias[n]) + res[m, n]) with acc[m, n] =
+// sum_k x[m, k] * q[n, k] accumulated in f32. The bf16 MFMA runs 16 times the f32 MFMA rate
+// on this chip, and every product fits it exactly: q (|q| <= 127: 7 bits) is exact in bf16,
+// and x is the exact sum of three bf16 pieces (bq_bf16x3.h), so each x * q is three exact
+// products (at most 15 significant bits) that three v_mfma_f32_16x16x32_bf16 add into one f32
+// accumulator: the accumulation is the only rounding before the per-channel scale, applied
+// once to the sum. The reference's order (the effective weight f32(q) * s rounded per element,
+// then f32 FMAs, kernels.ts:2695-2708) and this one are both within the f32-accumulation
+// bound (K + 2) 2^-24 sum |x * w| of the exact result on the effective weights.
 //
-// Tiles: BM x BN outputs a workgroup of WM x WN waves, each wave (BM / WM) x (BN / WN) in
-// 16 x 16 MFMA blocks. K goes in stages of 32 (one MFMA's K) through two LDS buffers: the
-// next stage's global loads (x as float4, the weight as 16-byte pieces) are issued before
-// the current stage's MFMAs and written to the other buffer after them, x as its three bf16
-// planes and q as bf16, so the MFMAs read ready operands. LDS rows are 64 bytes (32 bf16)
-// with the 16-byte chunk index XORed by bits 2..3 of the row: the 16 lanes that read one
-// fragment (16 rows, one chunk) then cover all 64 banks once.
+// The weight is the MFMA's first operand, so a lane's four results are four consecutive
+// outputs of one row (16-byte stores). K goes in chunks of 64. x is loaded so that the four
+// lanes g = l / 16 of a row take 64 contiguous bytes a load: lane (r = l % 16, g) holds values
+// 16 t + 4 g + (0..3), t = 0..3, of row r's chunk, and MFMA step h takes t = 2 h and 2 h + 1 in
+// both operands (the contracted index permuted alike in both).
 
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-typedef float v2f __attribute__((ext_vector_type(2)));
-
-// Byte offset of 16-byte chunk c of LDS row r, rows of CPR chunks (BK bf16): the chunk index
-// is XORed with the row bits that make the 16 rows of one fragment read cover all 64 banks.
-template <int CPR>
-__device__ __forceinline__ int w8_lds_off(int r, int c) {
-  if constexpr (CPR == 4) return r * 64 + ((c ^ ((r >> 2) & 3)) << 4);
-  else if constexpr (CPR == 8) return r * 128 + ((c ^ ((r >> 1) & 7)) << 4);
-  else return r * 256 + ((c ^ (r & 15)) << 4);
-}
-
-// Two floats to two bf16 (round to nearest even, v_cvt_pk_bf16_f32), packed low first.
-__device__ __forceinline__ uint32_t bf2(float a, float b) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f){a, b}, v2bf));
-}
-
-// The three bf16 planes of four floats: p1 = bf16(v), p2 = bf16(v - p1), p3 = v - p1 - p2.
-__device__ __forceinline__ void split3(float4 v, uint2& p1, uint2& p2, uint2& p3) {
-  const uint32_t a = bf2(v.x, v.y), b = bf2(v.z, v.w);
-  const float r0 = __fsub_rn(v.x, __uint_as_float(a << 16)), r1 = __fsub_rn(v.y, __uint_as_float(a & 0xffff0000u));
-  const float r2 = __fsub_rn(v.z, __uint_as_float(b << 16)), r3 = __fsub_rn(v.w, __uint_as_float(b & 0xffff0000u));
-  const uint32_t c = bf2(r0, r1), d = bf2(r2, r3);
-  const float t0 = __fsub_rn(r0, __uint_as_float(c << 16)), t1 = __fsub_rn(r1, __uint_as_float(c & 0xffff0000u));
-  const float t2 = __fsub_rn(r2, __uint_as_float(d << 16)), t3 = __fsub_rn(r3, __uint_as_float(d & 0xffff0000u));
-  p1 = make_uint2(a, b);
-  p2 = make_uint2(c, d);
-  p3 = make_uint2(bf2(t0, t1), bf2(t2, t3));
-}
-
-// Four signed bytes (low first) to four bf16, exactly: f32(q) has at most 7 significant
-// bits, so its bf16 is its upper half.
-__device__ __forceinline__ uint2 i8x4_bf16(uint32_t w) {
-  const float f0 = (float)(int)(int8_t)(w & 0xff), f1 = (float)(int)(int8_t)((w >> 8) & 0xff);
-  const float f2 = (float)(int)(int8_t)((w >> 16) & 0xff), f3 = (float)(int)(int8_t)(w >> 24);
-  return make_uint2(__builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u),
-                    __builtin_amdgcn_perm(__float_as_uint(f3), __float_as_uint(f2), 0x07060302u));
-}
+constexpr int W8_WAVES = 8;  // waves of a K-split workgroup
 
 struct W8P {
   const float* x;    // [M, K]
@@ -354,145 +311,360 @@ struct W8P {
   const float* res;  // [M, N] or null
   int act;
   float* out;        // [M, N]
+  int vec;           // N % 4 == 0 and every pointer 16-byte aligned: whole float4s
 };
 
-template <int BM, int BN, int WM, int WN, int BK>
-__global__ __launch_bounds__(WM * WN * 64) void w8a32_gemm_kernel(W8P p) {
-  static_assert(BK == 32 || BK == 64 || BK == 128, "K per stage");
-  constexpr int CPR = BK / 8;  // 16-byte chunks of an LDS row (BK bf16)
-  constexpr int T = WM * WN * 64;
-  constexpr int WTM = BM / WM, WTN = BN / WN;  // wave tile
-  constexpr int FM = WTM / 16, FN = WTN / 16;  // MFMA blocks a wave
-  static_assert(FM >= 1 && FN >= 1 && WTM % 16 == 0 && WTN % 16 == 0, "wave tile of whole 16x16 blocks");
-  constexpr int PLANE = BM * BK * 2;            // bytes of one bf16 plane of the x stage
-  constexpr int STAGE = 3 * PLANE + BN * BK * 2;  // x planes, then the weight
-  constexpr int NA = BM * (BK / 4);             // float4s of x a stage
-  constexpr int NW = BN * (BK / 16);            // 16-byte weight pieces a stage
-  constexpr int RA = (NA + T - 1) / T, RW = (NW + T - 1) / T;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * STAGE];
+// The plain f32 sum of one output. The split leaves NaN where x is infinite or rounds to a
+// bf16 infinity, so a sum that is not finite is taken again this way: an infinity, a NaN or
+// an overflow of the f32 sum itself then comes out as f32 arithmetic gives it.
+__device__ __attribute__((noinline)) float w8_dot_f32(const float* x, const int8_t* w, int K) {
+  float s = 0.f;
+  for (int k = 0; k < K; ++k) s = __fmaf_rn(x[k], (float)w[k], s);
+  return s;
+}
 
+// Outputs n .. n + 3 of row m from their sums.
+__device__ __forceinline__ void w8_store4(const W8P& p, int m, int n, v4f v) {
+  if (m >= p.M || n >= p.N) return;
+  if (!__builtin_isfinite(v[0] + v[1] + v[2] + v[3]))
+    for (int e = 0; e < 4 && n + e < p.N; ++e)
+      v[e] = w8_dot_f32(p.x + (size_t)m * p.K, p.W + (size_t)(n + e) * p.K, p.K);
+  const size_t o = (size_t)m * p.N + n;
+  if (p.vec) {
+    const float4 s = *reinterpret_cast<const float4*>(p.sW + n);
+    float4 y = make_float4(__fmul_rn(v[0], s.x), __fmul_rn(v[1], s.y), __fmul_rn(v[2], s.z), __fmul_rn(v[3], s.w));
+    if (p.bias) {
+      const float4 b = *reinterpret_cast<const float4*>(p.bias + n);
+      y = make_float4(__fadd_rn(y.x, b.x), __fadd_rn(y.y, b.y), __fadd_rn(y.z, b.z), __fadd_rn(y.w, b.w));
+    }
+    if (p.res) {
+      const float4 r = *reinterpret_cast<const float4*>(p.res + o);
+      y = make_float4(__fadd_rn(y.x, r.x), __fadd_rn(y.y, r.y), __fadd_rn(y.z, r.z), __fadd_rn(y.w, r.w));
+    }
+    *reinterpret_cast<float4*>(p.out + o) =
+        make_float4(activate(y.x, p.act), activate(y.y, p.act), activate(y.z, p.act), activate(y.w, p.act));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (n + e >= p.N) return;
+      float y = __fmul_rn(v[e], p.sW[n + e]);
+      if (p.bias) y = __fadd_rn(y, p.bias[n + e]);
+      if (p.res) y = __fadd_rn(y, p.res[o + e]);
+      p.out[o + e] = activate(y, p.act);
+    }
+  }
+}
+
+// A lane's 16 contiguous weights (words t = 0..3 of group g: values 16 g + 4 t + (0..3)) into
+// the order x is held in (word t of group g: values 16 t + 4 g + (0..3)): the 4 x 4 transpose
+// of words and lane groups, by two exchanges of half waves and two of 16-lane rows.
+__device__ __forceinline__ v4i w8_transpose(v4i w) {
+  typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+  const v2u a = __builtin_amdgcn_permlane32_swap((uint32_t)w[0], (uint32_t)w[2], false, false);
+  const v2u b = __builtin_amdgcn_permlane32_swap((uint32_t)w[1], (uint32_t)w[3], false, false);
+  const v2u c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const v2u d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  return (v4i){(int)c[0], (int)c[1], (int)d[0], (int)d[1]};
+}
+
+// Few rows: a workgroup owns 16 FM x 16 FN outputs over one of S slices of K, and its waves
+// split the slice (wave w takes chunks w, w + WAVES, ...), each straight from memory into
+// registers, PF chunks ahead; the waves' partial blocks meet through LDS in wave order, the
+// slices' through the workspace in slice order (`part` null: this workgroup takes every slice
+// in turn, which gives the same sums). As in the int8 GEMM's K split, no workgroup waits for
+// another: a tile's last one (its counter) adds the slices, runs the epilogue and clears the
+// counter; partials are device-scope relaxed atomics, complete before the counter's increment.
+//
+// What bounds it is the bytes a CU pulls through its L1, x above all (four bytes a value
+// against the weight's one): 16 rows of 4096 are 256 KB in every workgroup of a grid that only
+// splits N. Slices of K cut that, for the 2-3 us that the exchange of partials takes: 16 rows
+// against a 4096 x 4096 weight 13.5 us unsliced, 11.6 us as 64 tiles of 16 x 64 in 4 slices
+// (f32 MFMA on the unsplit rows, as below but for this K: 15.5 us). Against 32 x 64 tiles
+// staged through LDS: M = 17 35.8 -> 13.1 us, M = 64 36.2 -> 19.9, M = 256 47.8 -> 41.0.
+template <int FM, int FN, int PF>
+__global__ __launch_bounds__(W8_WAVES * 64) void w8a32_ksplit_kernel(W8P p, int S, int* cnt, uint64_t* part) {
+  constexpr int WAVES = W8_WAVES, T = WAVES * 64, ITEMS = FM * FN * 64, PER = (ITEMS + T - 1) / T;
+  __shared__ __attribute__((aligned(16))) v4f red[WAVES * ITEMS];
+  __shared__ int s_last;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / WN, wn = wave % WN;
-  const int tiles_m = (p.M + BM - 1) / BM, tiles_n = (p.N + BN - 1) / BN;
-  int bm, bn;
-  tile_of(xcd_order(blockIdx.x, gridDim.x), tiles_m, tiles_n, bm, bn);
-  const int m0 = bm * BM, n0 = bn * BN;
+  const int r = lane & 15, g = lane >> 4;
   const int K = p.K;
+  const int groups = part ? S : 1;  // workgroups of a tile
+  const int id = xcd_order(blockIdx.x, gridDim.x);
+  const int tiles_m = (p.M + 16 * FM - 1) / (16 * FM), tiles_n = (p.N + 16 * FN - 1) / (16 * FN);
+  int bm, bn;
+  tile_of(id / groups, tiles_m, tiles_n, bm, bn);
+  const int slice = id % groups;
+  const int m0 = bm * 16 * FM, n0 = bn * 16 * FN;
   const __amdgpu_buffer_rsrc_t rx = w_rsrc(p.x, (uint32_t)((size_t)p.M * K * 4));
   const __amdgpu_buffer_rsrc_t rw = w_rsrc(p.W, (uint32_t)((size_t)p.N * K));
-
-  float4 xa[RA];
-  v4i wq[RW];
-  auto load = [&](int kt) {
-    const int k0 = kt * BK;
+  uint32_t xo[FM], wo[FN];  // byte offsets of this lane's rows; a row past the edge stays out of range
 #pragma unroll
-    for (int r = 0; r < RA; ++r) {
-      const int i = tid + r * T;
-      const int row = i / (BK / 4), k = k0 + (i % (BK / 4)) * 4;
-      const bool ok = (NA % T == 0 || i < NA) && m0 + row < p.M && k < K;
-      xa[r] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
-                                             rx, ok ? (uint32_t)(((m0 + row) * K + k) * 4) : W_OOB, 0, 0));
+  for (int i = 0; i < FM; ++i) {
+    const int m = m0 + 16 * i + r;
+    xo[i] = m < p.M ? (uint32_t)(m * K + 4 * g) * 4u : W_OOB;
+  }
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int n = n0 + 16 * j + r;
+    wo[j] = n < p.N ? (uint32_t)(n * K + 16 * g) : W_OOB;
+  }
+  float4 xb[PF][FM][4];
+  v4i wb[PF][FN];
+  auto load_x = [&](int s, int c) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        xb[s][i][t] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                     rx, c * 64 + 16 * t < K ? xo[i] + (c * 64 + 16 * t) * 4 : W_OOB, 0, 0));
+  };
+  auto load_w = [&](int s, int j, int c) {
+    const uint32_t off = c * 64 + 16 * g < K ? wo[j] + c * 64 : W_OOB;
+    wb[s][j] = FM == 1 ? load_nt16(rw, off) : __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, off, 0, 0));
+  };
+  const int KT = (K + 63) / 64, per = (KT + S - 1) / S;
+  v4f sum[PER];
+  for (int q = 0; q < S / groups; ++q) {
+    const int c_begin = (slice + q) * per, c_end = min(KT, c_begin + per);
+    v4f acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < PF; ++s) {
+      const int c = c_begin + wave + s * WAVES;
+      if (c >= c_end) break;  // uniform across the wave
+#pragma unroll
+      for (int j = 0; j < FN; ++j) load_w(s, j, c);
+      load_x(s, c);
     }
+    __builtin_amdgcn_sched_barrier(0);  // every load above is issued before the first product
+    for (int c0 = c_begin + wave; c0 < c_end; c0 += WAVES * PF) {
 #pragma unroll
-    for (int r = 0; r < RW; ++r) {
-      const int i = tid + r * T;
-      const int row = i / (BK / 16), k = k0 + (i % (BK / 16)) * 16;
-      const bool ok = (NW % T == 0 || i < NW) && n0 + row < p.N && k < K;
-      wq[r] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
-                                         rw, ok ? (uint32_t)((n0 + row) * K + k) : W_OOB, 0, 0));
+      for (int s = 0; s < PF; ++s) {
+        const int c = c0 + s * WAVES, next = c + WAVES * PF;
+        if (c >= c_end) break;
+        Split8 a[2][FM];  // x is split first: its registers then take the chunk PF ahead
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < FM; ++i) a[h][i] = split8(xb[s][i][2 * h], xb[s][i][2 * h + 1]);
+        if (next < c_end) {
+          load_x(s, next);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          const v4i w = w8_transpose(wb[s][j]);
+          if (next < c_end) load_w(s, j, next);
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const v8bf b = i8x8_bf16((uint32_t)w[2 * h], (uint32_t)w[2 * h + 1]);
+#pragma unroll
+            for (int i = 0; i < FM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[h][i].p3, acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < FM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[h][i].p2, acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < FM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[h][i].p1, acc[i][j], 0, 0, 0);
+          }
+        }
+      }
+    }
+    if (q) __syncthreads();  // the previous slice's blocks have been read
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) red[((wave * FM + i) * FN + j) * 64 + lane] = acc[i][j];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int e = tid + u * T;
+      if (ITEMS % T == 0 || e < ITEMS) {
+        v4f v = red[e];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) v += red[w * ITEMS + e];
+        sum[u] = q ? sum[u] + v : v;
+      }
+    }
+  }
+  if (groups > 1) {
+    const int tile = bm * tiles_n + bn;
+    uint64_t* const mine = part + (size_t)(tile * S + slice) * ITEMS * 2;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int e = tid + u * T;
+      if (ITEMS % T == 0 || e < ITEMS)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          __hip_atomic_store(mine + h * ITEMS + e,
+                             (uint64_t)__float_as_uint(sum[u][2 * h]) | (uint64_t)__float_as_uint(sum[u][2 * h + 1]) << 32,
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every partial store of this lane has completed
+    __syncthreads();
+    if (tid == 0)
+      s_last = __hip_atomic_fetch_add(cnt + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == S - 1;
+    __syncthreads();
+    if (!s_last) return;  // uniform across the workgroup
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int e = tid + u * T;
+      if (ITEMS % T == 0 || e < ITEMS) {
+        v4f v = {0.f, 0.f, 0.f, 0.f};
+        const uint64_t* from = part + (size_t)tile * S * ITEMS * 2 + e;
+        for (int s0 = 0; s0 < S; s0 += 4) {  // four slices' loads in flight
+          uint64_t w[4][2];
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+              w[s][h] = s0 + s < S ? __hip_atomic_load(const_cast<uint64_t*>(from) + (size_t)((s0 + s) * 2 + h) * ITEMS,
+                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                   : 0;
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            if (s0 + s >= S) break;
+            const v4f x = {__uint_as_float((uint32_t)w[s][0]), __uint_as_float((uint32_t)(w[s][0] >> 32)),
+                           __uint_as_float((uint32_t)w[s][1]), __uint_as_float((uint32_t)(w[s][1] >> 32))};
+            v = s0 + s ? v + x : x;
+          }
+        }
+        sum[u] = v;
+      }
+    }
+    if (tid == 0) __hip_atomic_store(cnt + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int e = tid + u * T;
+    const int l = e & 63, j = (e >> 6) % FN, i = (e >> 6) / FN;
+    if (ITEMS % T == 0 || e < ITEMS) w8_store4(p, m0 + 16 * i + (l & 15), n0 + 16 * j + 4 * (l >> 4), sum[u]);
+  }
+}
+
+// Many rows: a workgroup of WAVES waves owns 16 FM WAVES x 16 FN outputs, each wave 16 FM
+// rows over all the columns. A wave's rows are its own, so x goes straight from memory into
+// registers and is split there once; the weight chunk, which the waves share, is expanded
+// to bf16 once a workgroup into one of two LDS buffers (128-byte rows, 16-byte pieces XORed by
+// row bits so that a fragment read's 16 rows cover all 64 banks), one barrier a chunk: the next
+// chunk's weights are expanded and stored between this chunk's MFMAs. 16 rows a wave keep the
+// registers at 128, four waves a SIMD, whose splits (5.5 VALU a value of x) then run under each
+// other's MFMAs; 32 rows a wave (two waves a SIMD) measured 10-40% slower, and so did
+// fragments read one at a time or all eight ahead. Against x staged through LDS as its three
+// planes: 6304 x 3072 x 768 114 -> 99 us, 6304 x 768 x 3072 138 -> 104, 2048^3 72 -> 53,
+// 4096^3 380 -> 334 us (1.23 PFLOP/s of bf16 products; a bf16 library product of 8192^3
+// runs at 1.13 here). MFMAs and splits alone would take about half of it.
+__device__ __forceinline__ int w8_lds_off(int row, int c) { return row * 128 + ((c ^ ((row >> 1) & 7)) << 4); }
+
+template <int FM, int FN, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 4) void w8a32_tile_kernel(W8P p) {
+  constexpr int BM = 16 * FM * WAVES, BN = 16 * FN, T = WAVES * 64;
+  constexpr int RW = BN * 4 / T;  // 16-byte weight pieces a thread and chunk
+  static_assert(RW * T == BN * 4, "whole pieces");
+  constexpr int STAGE = BN * 128;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * STAGE];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int K = p.K, KT = (K + 63) / 64;
+  int bm, bn;
+  tile_of(xcd_order(blockIdx.x, gridDim.x), (p.M + BM - 1) / BM, (p.N + BN - 1) / BN, bm, bn);
+  const int m0 = bm * BM + wave * 16 * FM, n0 = bn * BN;
+  const __amdgpu_buffer_rsrc_t rx = w_rsrc(p.x, (uint32_t)((size_t)p.M * K * 4));
+  const __amdgpu_buffer_rsrc_t rw = w_rsrc(p.W, (uint32_t)((size_t)p.N * K));
+  uint32_t xo[FM];  // byte offset of this lane's row and quad; a row past M stays out of range
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    const int m = m0 + 16 * i + r;
+    xo[i] = m < p.M ? (uint32_t)(m * K + 4 * g) * 4u : W_OOB;
+  }
+  float4 xb[2][FM][4];
+  v4i wq[RW];
+  auto load_x = [&](int s, int c) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        xb[s][i][t] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                     rx, c * 64 + 16 * t < K ? xo[i] + (c * 64 + 16 * t) * 4 : W_OOB, 0, 0));
+  };
+  auto load_w = [&](int c) {
+#pragma unroll
+    for (int e = 0; e < RW; ++e) {
+      const int i = tid + e * T, n = n0 + (i >> 2), k = c * 64 + (i & 3) * 16;
+      const uint32_t off = n < p.N && k < K ? (uint32_t)(n * K + k) : W_OOB;
+      wq[e] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, off, 0, 0));
     }
   };
-  auto store = [&](int buf) {
+  auto store_w = [&](int buf) {
     unsigned char* st = lds + buf * STAGE;
 #pragma unroll
-    for (int r = 0; r < RA; ++r) {
-      const int i = tid + r * T;
-      if (NA % T == 0 || i < NA) {
-        const int row = i / (BK / 4), c4 = i % (BK / 4);  // floats 4 c4 .. 4 c4 + 3: chunk c4 / 2, half c4 % 2
-        const int off = w8_lds_off<CPR>(row, c4 >> 1) + (c4 & 1) * 8;
-        uint2 p1, p2, p3;
-        split3(xa[r], p1, p2, p3);
-        *reinterpret_cast<uint2*>(st + off) = p1;
-        *reinterpret_cast<uint2*>(st + PLANE + off) = p2;
-        *reinterpret_cast<uint2*>(st + 2 * PLANE + off) = p3;
-      }
-    }
+    for (int e = 0; e < RW; ++e) {
+      const int i = tid + e * T, row = i >> 2, t = i & 3;  // values 16 t + 4 g + (0..3): group g's half t % 2 of step t / 2
 #pragma unroll
-    for (int r = 0; r < RW; ++r) {
-      const int i = tid + r * T;
-      if (NW % T == 0 || i < NW) {
-        const int row = i / (BK / 16), c0 = (i % (BK / 16)) * 2;  // 16 weights: chunks c0, c0 + 1
-        const uint2 a = i8x4_bf16((uint32_t)wq[r][0]), b = i8x4_bf16((uint32_t)wq[r][1]);
-        const uint2 c = i8x4_bf16((uint32_t)wq[r][2]), d = i8x4_bf16((uint32_t)wq[r][3]);
-        *reinterpret_cast<uint4*>(st + 3 * PLANE + w8_lds_off<CPR>(row, c0)) = make_uint4(a.x, a.y, b.x, b.y);
-        *reinterpret_cast<uint4*>(st + 3 * PLANE + w8_lds_off<CPR>(row, c0 + 1)) = make_uint4(c.x, c.y, d.x, d.y);
-      }
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<uint2*>(st + w8_lds_off(row, 2 * q + (t >> 1)) + (t & 1) * 8) = i8x4_bf16((uint32_t)wq[e][q]);
     }
   };
-
   v4f acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
-
-  const int KT = (K + BK - 1) / BK;
-  const int fr = lane & 15, fc = lane >> 4;  // a fragment lane's row in its block, and its 16-byte chunk
-  load(0);
-  store(0);
-  for (int kt = 0; kt < KT; ++kt) {
-    const int buf = kt & 1;
-    if (kt + 1 < KT) load(kt + 1);
-    __syncthreads();
-    const unsigned char* st = lds + buf * STAGE;
+  load_w(0);
+  load_x(0, 0);
+  store_w(0);
+  load_w(1);  // past K: zeros
+  auto chunk = [&](int c, int s) {
+    __syncthreads();  // chunk c's weights are stored; nobody reads the other buffer any more
+    load_x(s ^ 1, c + 1);
+    __builtin_amdgcn_sched_barrier(0);  // issued here, not sunk to its use
+    const unsigned char* st = lds + (c & 1) * STAGE;
+    constexpr int NB = 4;  // weight fragments read ahead of their products
 #pragma unroll
-    for (int ks = 0; ks < BK / 32; ++ks) {  // one MFMA K (32) at a time: chunks 4 ks .. 4 ks + 3
-      const int ch = ks * 4 + fc;
-      v8bf b[FN];
+    for (int h = 0; h < 2; ++h) {
+      v8bf b[NB];
+      Split8 a[FM];
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
-        b[j] = *reinterpret_cast<const v8bf*>(st + 3 * PLANE + w8_lds_off<CPR>(wn * WTN + j * 16 + fr, ch));
+      for (int j0 = 0; j0 < FN; j0 += NB) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const int off = w8_lds_off<CPR>(wm * WTM + i * 16 + fr, ch);
-        const v8bf a1 = *reinterpret_cast<const v8bf*>(st + off);
-        const v8bf a2 = *reinterpret_cast<const v8bf*>(st + PLANE + off);
-        const v8bf a3 = *reinterpret_cast<const v8bf*>(st + 2 * PLANE + off);
+        for (int j = 0; j < NB; ++j) b[j] = *reinterpret_cast<const v8bf*>(st + w8_lds_off(16 * (j0 + j) + r, 2 * g + h));
+        if (j0 == 0) {
 #pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a3, b[j], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b[j], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b[j], acc[i][j], 0, 0, 0);
+          for (int i = 0; i < FM; ++i) a[i] = split8(xb[s][i][2 * h], xb[s][i][2 * h + 1]);
         }
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+            acc[i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i].p3, acc[i][j0 + j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+            acc[i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i].p2, acc[i][j0 + j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int i = 0; i < FM; ++i)
+            acc[i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i].p1, acc[i][j0 + j], 0, 0, 0);
+      }
+      if (h == 0) {
+        store_w((c & 1) ^ 1);
+        load_w(c + 2);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if (kt + 1 < KT) store(buf ^ 1);
-  }
-
-  // Epilogue: block (i, j) register r of lane l is row 4 (l / 16) + r, column l % 16.
-  float sc[FN], bi[FN];
-#pragma unroll
-  for (int j = 0; j < FN; ++j) {
-    const int n = n0 + wn * WTN + j * 16 + fr;
-    sc[j] = n < p.N ? p.sW[n] : 0.f;
-    bi[j] = (p.bias && n < p.N) ? p.bias[n] : 0.f;
+  };
+  for (int c = 0; c < KT; c += 2) {
+    chunk(c, 0);
+    if (c + 1 < KT) chunk(c + 1, 1);
   }
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + wm * WTM + i * 16 + fc * 4 + r;
-      if (m >= p.M) continue;
-#pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const int n = n0 + wn * WTN + j * 16 + fr;
-        if (n >= p.N) continue;
-        float v = __fmul_rn(acc[i][j][r], sc[j]);
-        if (p.bias) v = __fadd_rn(v, bi[j]);
-        if (p.res) v = __fadd_rn(v, p.res[(size_t)m * p.N + n]);
-        p.out[(size_t)m * p.N + n] = activate(v, p.act);
-      }
-    }
+    for (int j = 0; j < FN; ++j) w8_store4(p, m0 + 16 * i + r, n0 + 16 * j + 4 * g, acc[i][j]);
 }
 
 // w[n, k] = f32(q[n, k]) * s[n] (one rounding), four elements a thread.
@@ -519,13 +691,6 @@ static void launch_gemv_w8a32(const float* x, const int8_t* W, int m, int n, int
   constexpr int RPW = 2;
   const unsigned grid = (unsigned)((n + WA_WAVES * RPW - 1) / (WA_WAVES * RPW));
   const int64_t M = m, K = k;
-  if (m >= WA_MFMA_MIN_M) {
-    const unsigned g2 = (unsigned)((n + WM_ROWS - 1) / WM_ROWS);
-    if (K <= 2048) gemv_w8a32_mfma_kernel<4><<<g2, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-    else if (K <= 4096) gemv_w8a32_mfma_kernel<8><<<g2, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-    else gemv_w8a32_mfma_kernel<16><<<g2, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-    return;
-  }
   const int64_t kc = K <= 1024 ? 1 : K <= 2048 ? 2 : K <= 4096 ? 4 : 8;  // the kernel's KC
   if (M * kc * 1024 <= WA_XLDS) {
     if (K <= 1024) (m == 1 ? gemv_w8a32_kernel<1, RPW, true, WA_XLDS, true> : gemv_w8a32_kernel<1, RPW, true>)<<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
@@ -546,15 +711,34 @@ static void launch_gemv_w8a32(const float* x, const int8_t* W, int m, int n, int
   }
 }
 
-template <int BM, int BN, int WM, int WN, int BK>
-static void launch_w8a32_tiled(const W8P& p, hipStream_t st) {
+struct W8Ws {
+  void* ptr;
+  size_t bytes;
+};
+template <int FM, int FN, int PF>
+static void launch_w8a32_ksplit(const W8P& p, const W8Ws& ws, hipStream_t st) {
+  const int tiles = ((p.M + 16 * FM - 1) / (16 * FM)) * ((p.N + 16 * FN - 1) / (16 * FN));
+  const int KT = (p.K + 63) / 64;
+  int S = std::max(1, std::min(256 / tiles, KT / W8_WAVES));
+  const int per = (KT + S - 1) / S;
+  S = (KT + per - 1) / per;  // no empty slice
+  if ((size_t)tiles * S * FM * FN * 1024 > W8_WS_BYTES - W8_CNT_BYTES || tiles * 4 > (int)W8_CNT_BYTES) S = 1;
+  const bool split = S > 1 && ws.ptr && ws.bytes >= W8_WS_BYTES;
+  int* cnt = split ? static_cast<int*>(ws.ptr) : nullptr;
+  uint64_t* part = split ? reinterpret_cast<uint64_t*>(static_cast<char*>(ws.ptr) + W8_CNT_BYTES) : nullptr;
+  w8a32_ksplit_kernel<FM, FN, PF><<<tiles * (split ? S : 1), W8_WAVES * 64, 0, st>>>(p, S, cnt, part);
+}
+
+template <int FM, int FN, int WAVES>
+static void launch_w8a32_tile(const W8P& p, hipStream_t st) {
+  constexpr int BM = 16 * FM * WAVES, BN = 16 * FN;
   const unsigned tiles = (unsigned)(((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN));
-  w8a32_gemm_kernel<BM, BN, WM, WN, BK><<<tiles, WM * WN * 64, 0, st>>>(p);
+  w8a32_tile_kernel<FM, FN, WAVES><<<tiles, WAVES * 64, 0, st>>>(p);
 }
 
 static int w8a32_common(const char* what, const float* x, const int8_t* W, int64_t M, int64_t N, int64_t K,
                         const float* sW, const float* bias, const float* res, int act, float* out, int max_m,
-                        bq_stream_t stream) {
+                        const W8Ws& ws, bq_stream_t stream) {
   if (M < 0 || N < 0 || K < 0) return set_error(BQ_ERR_ARG, "%s: negative size", what);
   if (M == 0 || N == 0) return BQ_OK;
   if (M > max_m)
@@ -567,21 +751,41 @@ static int w8a32_common(const char* what, const float* x, const int8_t* W, int64
   if (((uintptr_t)x & 15) || ((uintptr_t)W & 15)) return set_error(BQ_ERR_ARG, "%s: x and W must be 16-byte aligned", what);
   if (act < BQ_ACT_NONE || act > BQ_ACT_GELU) return set_error(BQ_ERR_ARG, "%s: bad activation %d", what, act);
   hipStream_t st = (hipStream_t)stream;
-  if (M <= WA_MMAX && K <= 8192) {
+  if (M <= WA_MPW && K <= 8192) {
     launch_gemv_w8a32(x, W, (int)M, (int)N, (int)K, sW, bias, res, act, out, st);
     return check_launch(what);
   }
-  W8P p{x, W, (int)M, (int)N, (int)K, sW, bias, res, act, out};
-  // Measured (4096 x 4096 weight; M = 17 .. 256 and 1024, 4096, ViT-B's 6304-row shapes):
-  // skinny 32 x 64 tiles with 128-deep K stages while M <= 256 (37-53 us, against 57-128
-  // with 32-deep stages: fewer stage round trips), 128 x 128 tiles once they give a
-  // workgroup per CU (4096^3: 384 us), 64 x 64 with 64-deep stages between.
-  const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128);
-  const int pick = M <= 256 ? 2 : t128 >= 256 ? 1 : 3;
-  switch (pick) {
-    case 1: launch_w8a32_tiled<128, 128, 2, 2, 32>(p, st); break;
-    case 2: launch_w8a32_tiled<32, 64, 1, 4, 128>(p, st); break;
-    default: launch_w8a32_tiled<64, 64, 2, 2, 64>(p, st); break;
+  const uintptr_t ptrs = (uintptr_t)sW | (uintptr_t)bias | (uintptr_t)res | (uintptr_t)out;
+  W8P p{x, W, (int)M, (int)N, (int)K, sW, bias, res, act, out, N % 4 == 0 && (ptrs & 15) == 0};
+  // The K-split kernel up to 511 tiles of 32 x 128 (2 a CU; 512 x 4096 x 4096 is 76 us there
+  // and 67 in the tiled one, 1024^3 15 and 22), its tile the largest that with its slices still
+  // gives the chip's CUs a workgroup each: 16 x 64 for 16 rows of 4096 x 4096 (16 x 32 12.8 us
+  // against 11.6) but 16 x 32 at 2048 x 2048 (16 x 64 8.1 us against 7.4); 32 x 128 from 160
+  // workgroups on (200 x 3072 x 768, 168 workgroups: 12.8 us, 17.5 in 336 of 32 x 64). Few rows
+  // of a short K stay with the f32 MFMA, which needs no split of x and no exchange (12 x 3000 x
+  // 1520 6.4 us against 7.6; at 16 x 2048 x 2048 8.5 against 7.4). Tiled: 128 x 128 workgroups
+  // where they fill the chip evenly (2048^3 55 us against 59 in 64 x 128), else 64 x 128
+  // (6304 x 768 x 3072, 300 tiles of 128 x 128: 108 us against 122).
+  const auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  // workgroups a K-split tile shape can fill: its tiles times the slices of at least a chunk a wave
+  const auto fill = [&](int fm, int fn) { return tiles(16 * fm, 16 * fn) * std::max<int64_t>(1, (K + 63) / 64 / W8_WAVES); };
+  if (M <= WA_MMAX) {
+    if (K <= 1024 || (K <= 2048 && M <= 12)) {
+      const unsigned grid = (unsigned)((N + WM_ROWS - 1) / WM_ROWS);
+      gemv_w8a32_mfma_kernel<4><<<grid, WA_WAVES * 64, 0, st>>>(x, W, (int)M, (int)N, (int)K, sW, bias, res, act, out);
+      return check_launch(what);
+    }
+    if (fill(1, 4) >= 256) launch_w8a32_ksplit<1, 4, 2>(p, ws, st);
+    else if (fill(1, 2) >= 256) launch_w8a32_ksplit<1, 2, 4>(p, ws, st);
+    else launch_w8a32_ksplit<1, 1, 4>(p, ws, st);
+  } else if (tiles(32, 128) < 512) {
+    if (M > 32 && fill(2, 8) >= 160) launch_w8a32_ksplit<2, 8, 1>(p, ws, st);
+    else if (fill(2, 4) >= 256) launch_w8a32_ksplit<2, 4, 2>(p, ws, st);
+    else launch_w8a32_ksplit<2, 2, 2>(p, ws, st);
+  } else {
+    const int64_t t = tiles(128, 128);
+    if (t >= 512 || (t >= 192 && t <= 256)) launch_w8a32_tile<1, 8, 8>(p, st);
+    else launch_w8a32_tile<1, 8, 4>(p, st);
   }
   return check_launch(what);
 }
@@ -595,12 +799,21 @@ extern "C" {
 int bq_gemv_w8a32(const float* x, const int8_t* W, int64_t M, int64_t N, int64_t K, const float* sW,
                   const float* bias, int act, float* out, bq_stream_t stream) {
   if (K > 8192) return set_error(BQ_ERR_UNSUPPORTED, "bq_gemv_w8a32: K=%lld > 8192", (long long)K);
-  return w8a32_common("bq_gemv_w8a32", x, W, M, N, K, sW, bias, nullptr, act, out, WA_MMAX, stream);
+  return w8a32_common("bq_gemv_w8a32", x, W, M, N, K, sW, bias, nullptr, act, out, WA_MMAX, W8Ws{nullptr, 0},
+                      stream);
 }
 
 int bq_linear_w8a32(const float* x, const int8_t* W, int64_t M, int64_t N, int64_t K, const float* sW,
                     const float* bias, const float* residual, int act, float* out, bq_stream_t stream) {
-  return w8a32_common("bq_linear_w8a32", x, W, M, N, K, sW, bias, residual, act, out, 0x7fffffff, stream);
+  return w8a32_common("bq_linear_w8a32", x, W, M, N, K, sW, bias, residual, act, out, 0x7fffffff,
+                      W8Ws{nullptr, 0}, stream);
+}
+
+int bq_linear_w8a32_ws(const float* x, const int8_t* W, int64_t M, int64_t N, int64_t K, const float* sW,
+                       const float* bias, const float* residual, int act, float* out, void* ws, size_t ws_bytes,
+                       bq_stream_t stream) {
+  return w8a32_common("bq_linear_w8a32_ws", x, W, M, N, K, sW, bias, residual, act, out, 0x7fffffff,
+                      W8Ws{ws, ws_bytes}, stream);
 }
 
 int bq_dequant_i8(const int8_t* q, int64_t N, int64_t K, const float* s, float* w, bq_stream_t stream) {

@@ -366,8 +366,8 @@ def linear_w8a32(x: torch.Tensor, w8: Int8Weight, bias=None, act=ACT_NONE, resid
         if tuple(residual.shape[:-1]) != tuple(lead) or residual.shape[-1] != N:
             raise RuntimeError(f"residual shape {tuple(residual.shape)} != output {(*lead, N)}")
         r = residual.reshape(M, N).float().contiguous()
-    check(lib().bq_linear_w8a32(x2.data_ptr(), w8.q.data_ptr(), M, N, K, w8.s.data_ptr(), _ptr(b), _ptr(r), act,
-                                out.data_ptr(), _stream(x2)))
+    check(lib().bq_linear_w8a32_ws(x2.data_ptr(), w8.q.data_ptr(), M, N, K, w8.s.data_ptr(), _ptr(b), _ptr(r), act,
+                                   out.data_ptr(), *_ws_args(x2.device), _stream(x2)))
     return out.reshape(*lead, N)
 
 

@@ -422,11 +422,12 @@ int bq_se_gate_nhwc(const float* x, int64_t N, int64_t HW, int64_t C, const floa
 
 /* Weight-only int8 (W8A32) Linear, any M: f32 x [M, K] against int8 W [N, K] with
  * per-channel sW [N]; out f32 [M, N] = act(y + bias[n] + residual[m, n]) with y the f32 sum
- * over k of x * f32(q) * sW[n] (bias, residual nullable; residual f32 [M, N]). M <= 16 (K <=
- * 8192): wave-reduction GEMV kernels, the effective weight f32(f32(q) * sW[n]) per element
- * and f32 FMA / f32-MFMA accumulation, as the reference. Otherwise a tiled bf16-MFMA kernel:
- * q is exact in bf16 and each x is split exactly into three bf16 pieces, so every product is
- * exact; the f32 accumulation is the only rounding before y = fl(sum * sW[n]). Either way
+ * over k of x * f32(q) * sW[n] (bias, residual nullable; residual f32 [M, N]). M <= 4 (K <=
+ * 8192): a wave-reduction GEMV, the effective weight f32(f32(q) * sW[n]) per element and f32
+ * FMA accumulation, as the reference; M <= 16 over a short K: the same weights on the f32 MFMA.
+ * Otherwise bf16-MFMA kernels: q is exact in bf16 and each x is split exactly into three bf16
+ * pieces, so every product is exact; the f32 accumulation is the only rounding before
+ * y = fl(sum * sW[n]) (a sum that comes out infinite or NaN is taken again in plain f32). Either way
  * every output is within (K + 2) 2^-24 sum_k |x * w| + 2^-24 |y| of the exact result on the
  * effective weights w = f32(q) * sW. The int8 weight is read inside the kernel: no f32 copy
  * of it is written. K % 16 == 0; x and W 16-byte aligned; x and W each < 2 GiB.
@@ -436,6 +437,13 @@ int bq_se_gate_nhwc(const float* x, int64_t N, int64_t HW, int64_t C, const floa
  * borch_webgpu/_stream.py:61-66). */
 int bq_linear_w8a32(const float* x, const int8_t* W, int64_t M, int64_t N, int64_t K, const float* sW,
                     const float* bias, const float* residual, int act, float* out, bq_stream_t stream);
+
+/* bq_linear_w8a32 with a workspace (ws of bq_gemm_ws_bytes() bytes, zero-filled once and shared
+ * with bq_gemm_i8's calls on the same stream; nullable): few rows over a long K run as slices of
+ * K on more workgroups. The same bits with and without it. */
+int bq_linear_w8a32_ws(const float* x, const int8_t* W, int64_t M, int64_t N, int64_t K, const float* sW,
+                       const float* bias, const float* residual, int act, float* out, void* ws, size_t ws_bytes,
+                       bq_stream_t stream);
 
 /* bq_linear_w8a32's decode-shape kernels alone (M <= 16, K <= 8192, no residual); the same
  * results. Kept for callers bound to it. */
