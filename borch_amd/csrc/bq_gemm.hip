@@ -583,8 +583,11 @@ __device__ __forceinline__ void gemm_tile(const GemmP& p, const int L,
   const bool has_out = p.out != nullptr;
   const bool fast = p.vec_ok && !p.acc && (p.q_out ? FASTQ && !p.amax : has_out) &&
                     (long long)BM * p.N * 4 < (1ll << 31);
+  // Rows that are no whole float4s (N % 4 != 0, or an unaligned output), the f32 output alone:
+  // the same stores with one column a lane, so that each takes 256 contiguous bytes of a row.
+  const bool narrow = !p.vec_ok && !p.acc && !p.q_out && has_out && (long long)BM * p.N * 4 < (1ll << 31);
   const int tile_rows = min(BM, p.M - m0);
-  const uint32_t tile_bytes = fast ? (uint32_t)((long long)tile_rows * p.N * 4) : 0u;
+  const uint32_t tile_bytes = fast || narrow ? (uint32_t)((long long)tile_rows * p.N * 4) : 0u;
   const __amdgpu_buffer_rsrc_t r_out = make_rsrc(has_out ? p.out + (size_t)m0 * p.N : p.out, has_out ? tile_bytes : 0u);
   const __amdgpu_buffer_rsrc_t r_res = make_rsrc(has_r ? p.res + (size_t)m0 * p.N : p.res, has_r ? tile_bytes : 0u);
   const __amdgpu_buffer_rsrc_t r_q = make_rsrc(p.q_out ? p.q_out + (size_t)m0 * p.N : p.q_out,
@@ -636,6 +639,58 @@ __device__ __forceinline__ void gemm_tile(const GemmP& p, const int L,
       if constexpr (AMAX) {  // rows past M are computed (and dropped) but must not count
         if (m0 + rl + k * ROWS_PER_STORE < p.M)
           amax = fmaxf(amax, fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fmaxf(fabsf(o.z), fabsf(o.w))));
+      }
+    }
+  };
+  // The 32 rows of a slice (tile rows rl .. rl + 31) from the patch, eight at a time: their LDS
+  // reads and residual loads together, no per-row test (rows past M fall out of the resource),
+  // the activation's branch once. The general path below takes a branch and an LDS round trip
+  // an element, with one wave a SIMD to hide them: 1000 x 2999 x 1568 26.2 us, here 13.4 (as
+  // N = 3000); 4095 x 4095 x 512 41.0 -> 22.8; 100 x 1001 x 1008 8.3 -> 5.7.
+  auto narrow_rows = [&]<bool RES>(int rl) __attribute__((always_inline)) {
+    constexpr int CW = WTN < 64 ? WTN : 64, RS = 64 / CW, NR = 8;  // columns and rows of a store, rows a batch
+#pragma unroll 1
+    for (int cc = 0; cc < WTN; cc += CW) {
+      const int nc = wn * WTN + cc + lane % CW;  // this lane's column of the tile
+      if (n0 + nc >= p.N) continue;
+      const float sw1 = s_sw[nc], b1 = s_b[nc];
+#pragma unroll 1
+      for (int rr = lane / CW; rr < 32; rr += NR * RS) {
+        const uint32_t voff = ((uint32_t)(rl + rr) * (uint32_t)p.N + (uint32_t)(n0 + nc)) * 4u;
+        const uint32_t step = (uint32_t)(RS * p.N) * 4u;
+        float o[NR], rv[NR];
+        if constexpr (RES) {
+#pragma unroll
+          for (int k = 0; k < NR; ++k)
+            rv[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r_res, voff + k * step, 0, 0));
+        }
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+          const int a = patch[(rr + k * RS) * PITCH + cc + lane % CW];
+          o[k] = __fadd_rn(__fmul_rn(__fmul_rn((float)a, s_sa[rl + rr + k * RS]), sw1), b1);
+          if constexpr (RES) o[k] = __fadd_rn(o[k], rv[k]);
+        }
+        if (p.act == BQ_ACT_RELU) {
+#pragma unroll
+          for (int k = 0; k < NR; ++k) o[k] = o[k] > 0.f ? o[k] : 0.f;
+        } else if (p.act == BQ_ACT_SILU) {
+#pragma unroll
+          for (int k = 0; k < NR; ++k) o[k] = silu(o[k]);
+        } else if (p.act == BQ_ACT_GELU) {
+#pragma unroll 1
+          for (int k = 0; k < NR; k += 4) {
+            const float4 y = gelu4(k ? make_float4(o[4], o[5], o[6], o[7]) : make_float4(o[0], o[1], o[2], o[3]));
+            if (k) { o[4] = y.x; o[5] = y.y; o[6] = y.z; o[7] = y.w; }
+            else { o[0] = y.x; o[1] = y.y; o[2] = y.z; o[3] = y.w; }
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < NR; ++k) store_wt4(r_out, voff + k * step, __float_as_uint(o[k]));
+        if (p.amax) {  // rows past M are computed (and dropped) but must not count
+#pragma unroll
+          for (int k = 0; k < NR; ++k)
+            if (m0 + rl + rr + k * RS < p.M) amax = fmaxf(amax, fabsf(o[k]));
+        }
       }
     }
   };
@@ -741,6 +796,9 @@ __device__ __forceinline__ void gemm_tile(const GemmP& p, const int L,
 #pragma unroll 1
         for (int rr = 0; rr < 32; rr += ROWS_PER_STORE) store_row(rr, make_float4(0.f, 0.f, 0.f, 0.f), false);
       }
+    } else if (narrow) {
+      if (has_r) narrow_rows.template operator()<true>(wm * WTM + i * 32);
+      else narrow_rows.template operator()<false>(wm * WTM + i * 32);
     } else if (!p.vec_ok) {
 #pragma unroll 1
       for (int rr = 0; rr < 32; rr += ROWS_PER_STORE) {
