@@ -93,6 +93,65 @@ __global__ __launch_bounds__(T) void quantize_rows_kernel(const float* __restric
   }
 }
 
+// The rows of a Linear whose width is no multiple of 16: x f32 [M, K], read at 4-byte alignment
+// (a 16-byte load needs no more), into q [M, Kp] with zeros from K on, in the one pass that the
+// torch pad before it took two kernels more for (1000 x 1555: 13.7 us as fill, copy and
+// quantize_rows_kernel). Rows in registers up to NV * 4 * T values; NV == 0 reads them twice.
+typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ float4 row4(const float* xr, int k, int K) {
+  if (k + 3 < K) {
+    const float4_u v = *reinterpret_cast<const float4_u*>(xr + k);
+    return make_float4(v[0], v[1], v[2], v[3]);
+  }
+  return make_float4(k < K ? xr[k] : 0.f, k + 1 < K ? xr[k + 1] : 0.f, k + 2 < K ? xr[k + 2] : 0.f, 0.f);
+}
+
+template <int NV, int T>
+__global__ __launch_bounds__(T) void quantize_rows_pad_kernel(const float* __restrict__ x, int K, int Kp,
+                                                              int8_t* __restrict__ q, float* __restrict__ s) {
+  __shared__ float red[T / 64];
+  const size_t row = blockIdx.x;
+  const float* xr = x + row * (size_t)K;
+  int8_t* qr = q + row * (size_t)Kp;
+  const int t = threadIdx.x;
+  auto peak4 = [](float m, float4 v) {
+    return fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+  };
+  float m = 0.f;
+  if constexpr (NV > 0) {
+    float4 v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      v[i] = row4(xr, (t + i * T) * 4, K);
+      m = peak4(m, v[i]);
+    }
+    const float sc = scale_of(block_max<T>(m, red));
+    if (t == 0) s[row] = sc;
+    const Quantizer qz(sc);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int k = (t + i * T) * 4;
+      if (k < Kp) *reinterpret_cast<uint32_t*>(qr + k) = qz.pack(v[i]);
+    }
+  } else {
+    for (int k = t * 4; k < K; k += T * 4) m = peak4(m, row4(xr, k, K));
+    const float sc = scale_of(block_max<T>(m, red));
+    if (t == 0) s[row] = sc;
+    const Quantizer qz(sc);
+    for (int k = t * 4; k < Kp; k += T * 4) *reinterpret_cast<uint32_t*>(qr + k) = qz.pack(row4(xr, k, K));
+  }
+}
+
+// The same rows as f32 [M, Kp] with zeros from K on.
+__global__ __launch_bounds__(256) void pad_rows_kernel(const float* __restrict__ x, int64_t M, int K, int Kp,
+                                                       float* __restrict__ y) {
+  const int k = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (k >= Kp) return;
+  for (int64_t row = blockIdx.y; row < M; row += gridDim.y)
+    *reinterpret_cast<float4*>(y + row * Kp + k) = row4(x + row * K, k, K);
+}
+
 // One wave per row, QW_WAVES rows per block, for rows of up to NV * 256 floats (NV <= 4): every lane
 // loads its NV float4 (coalesced: lane l reads bytes [16 l, 16 l + 16) of each 1 KB run)
 // before any arithmetic, so a wave has NV KB in flight; the max is a wave reduction (no
@@ -586,6 +645,41 @@ int bq_quantize_rows(const float* x, int64_t M, int64_t K, int8_t* q, float* s, 
 int bq_quantize_rows_act(const float* x, int64_t M, int64_t K, int act, int8_t* q, float* s, float* y,
                          bq_stream_t stream) {
   return launch_rows(x, M, K, q, s, (hipStream_t)stream, "bq_quantize_rows_act", act, y);
+}
+
+int bq_quantize_rows_padded(const float* x, int64_t M, int64_t K, int64_t Kp, int8_t* q, float* s,
+                            bq_stream_t stream) {
+  const char* what = "bq_quantize_rows_padded";
+  if (M < 0 || K < 0 || Kp < K) return set_error(BQ_ERR_ARG, "%s: bad sizes M=%lld K=%lld Kp=%lld", what, (long long)M, (long long)K, (long long)Kp);
+  if (M == 0) return BQ_OK;
+  if ((!x && K > 0) || !q || !s) return set_error(BQ_ERR_ARG, "%s: null pointer", what);
+  if (M > 0x7fffffff || Kp > 0x7ffffff0) return set_error(BQ_ERR_ARG, "%s: size too large", what);
+  if (Kp % 4 || ((uintptr_t)q & 3) || ((uintptr_t)x & 3))
+    return set_error(BQ_ERR_UNSUPPORTED, "%s: Kp %% 4 == 0 and 4-byte aligned x and q", what);
+  auto go = [&](auto kernel, int threads) {
+    kernel<<<dim3((unsigned)M), dim3(threads), 0, (hipStream_t)stream>>>(x, (int)K, (int)Kp, q, s);
+  };
+  if (Kp <= 256) go(quantize_rows_pad_kernel<1, 64>, 64);  // short rows: one wave a row
+  else if (Kp <= 512) go(quantize_rows_pad_kernel<2, 64>, 64);
+  else if (Kp <= 1024) go(quantize_rows_pad_kernel<1, 256>, 256);
+  else if (Kp <= 2048) go(quantize_rows_pad_kernel<2, 256>, 256);
+  else if (Kp <= 4096) go(quantize_rows_pad_kernel<4, 256>, 256);
+  else if (Kp <= 8192) go(quantize_rows_pad_kernel<8, 256>, 256);
+  else go(quantize_rows_pad_kernel<0, 256>, 256);
+  return check_launch(what);
+}
+
+int bq_pad_rows_f32(const float* x, int64_t M, int64_t K, int64_t Kp, float* y, bq_stream_t stream) {
+  const char* what = "bq_pad_rows_f32";
+  if (M < 0 || K < 0 || Kp < K) return set_error(BQ_ERR_ARG, "%s: bad sizes M=%lld K=%lld Kp=%lld", what, (long long)M, (long long)K, (long long)Kp);
+  if (M == 0 || Kp == 0) return BQ_OK;
+  if ((!x && K > 0) || !y) return set_error(BQ_ERR_ARG, "%s: null pointer", what);
+  if (Kp > 0x7ffffff0) return set_error(BQ_ERR_ARG, "%s: size too large", what);
+  if (Kp % 4 || ((uintptr_t)y & 15) || ((uintptr_t)x & 3))
+    return set_error(BQ_ERR_UNSUPPORTED, "%s: Kp %% 4 == 0, y 16-byte and x 4-byte aligned", what);
+  const dim3 grid((unsigned)((Kp / 4 + 255) / 256), (unsigned)(M < 65535 ? M : 65535));
+  pad_rows_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(x, M, (int)K, (int)Kp, y);
+  return check_launch(what);
 }
 
 int bq_quantize_weight_per_channel(const float* w, int64_t N, int64_t K, int8_t* q, float* s,

@@ -118,6 +118,20 @@ def quantize_rows(x: torch.Tensor, act: int = ACT_NONE, want_y: bool = False):
     return q, s
 
 
+def quantize_rows_padded(x: torch.Tensor, kpad: int):
+    """``quantize_rows`` of f32 ``[M, K]`` into ``q int8 [M, kpad]`` with zeros from K on
+    (bq_quantize_rows_padded): a Linear's input at its packed weight's width."""
+    x = _f32c(x)
+    require_device(x.device)
+    if x.dim() != 2:
+        raise ValueError("quantize_rows_padded wants a 2-D tensor")
+    M, K = x.shape
+    q = torch.empty((M, kpad), dtype=torch.int8, device=x.device)
+    s = torch.empty((M,), dtype=torch.float32, device=x.device)
+    check(lib().bq_quantize_rows_padded(x.data_ptr(), M, K, kpad, q.data_ptr(), s.data_ptr(), _stream(x)))
+    return q, s
+
+
 def quantize_weight_per_channel(w: torch.Tensor):
     """Per-output-channel int8 of a Linear weight ``[N, K]`` (quant.ts:23-53)."""
     w = _f32c(w)
@@ -356,7 +370,9 @@ def linear_w8a32(x: torch.Tensor, w8: Int8Weight, bias=None, act=ACT_NONE, resid
     lead = x.shape[:-1]
     x2 = _f32c(x.reshape(-1, x.shape[-1]))
     if w8.kpad != w8.in_features:
-        x2 = torch.nn.functional.pad(x2, (0, w8.kpad - w8.in_features))
+        xp = torch.empty((x2.shape[0], w8.kpad), dtype=torch.float32, device=x2.device)
+        check(lib().bq_pad_rows_f32(x2.data_ptr(), x2.shape[0], w8.in_features, w8.kpad, xp.data_ptr(), _stream(x2)))
+        x2 = xp
     M, K = x2.shape
     N = w8.out_features
     out = torch.empty((M, N), dtype=torch.float32, device=x.device)
@@ -721,9 +737,12 @@ def linear(x: torch.Tensor, w8: Int8Weight, bias=None, act=ACT_NONE, residual=No
             f"mat1 and mat2 shapes cannot be multiplied ({a} and {w8.in_features}x{w8.out_features})")
     lead = x.shape[:-1]
     x2 = x.reshape(-1, x.shape[-1])
-    if w8.kpad != w8.in_features:
-        x2 = torch.nn.functional.pad(x2, (0, w8.kpad - w8.in_features))
     r = None if residual is None else residual.reshape(-1, w8.out_features)
+    if w8.kpad != w8.in_features:
+        if not w8.per_tensor:  # the quantizer writes the padding
+            qa, sa = quantize_rows_padded(x2, w8.kpad)
+            return gemm_i8(qa, w8.q, sa, w8.s, bias, act, residual=r).reshape(*lead, w8.out_features)
+        x2 = torch.nn.functional.pad(x2, (0, w8.kpad - w8.in_features))
     if x2.shape[0] <= 4 and pre_act == ACT_NONE and not w8.per_tensor:
         return linear_rows(x2, w8, bias, act, r).reshape(*lead, w8.out_features)
     qa, sa = quantize_tensor(x2) if w8.per_tensor else quantize_rows(x2, pre_act)
