@@ -36,7 +36,8 @@ def _ptr(t):
 
 
 def _stream(t: torch.Tensor):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current stream's handle on ``t``'s device, without a Stream object (2 us a call)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 # The split-K workspaces of bq_gemm_i8 / bq_conv2d_i8_nhwc(_q) (bq_gemm_ws_bytes): one
@@ -69,7 +70,11 @@ def split_workspace(device: torch.device, stream=None):
 
 def _ws_args(device):
     """(pointer, bytes) of the current stream's split-K workspace, or (None, 0) (unsplit)."""
-    ws = split_workspace(device)
+    ws = None
+    if device.index is not None:  # one that is there already
+        ws = _SPLIT_WS.get((device.index, torch._C._cuda_getCurrentRawStream(device.index)))
+    if ws is None:
+        ws = split_workspace(device)
     return (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
 
 
@@ -86,6 +91,8 @@ def _vec(t, n: int, name: str):
         return None
     if t.numel() != n:
         raise ValueError(f"{name}: expected {n} values, got {t.numel()}")
+    if t.dtype == torch.float32 and t.is_contiguous():
+        return t
     return t.detach().reshape(-1).float().contiguous()
 
 
@@ -736,15 +743,17 @@ def linear(x: torch.Tensor, w8: Int8Weight, bias=None, act=ACT_NONE, residual=No
         raise RuntimeError(
             f"mat1 and mat2 shapes cannot be multiplied ({a} and {w8.in_features}x{w8.out_features})")
     lead = x.shape[:-1]
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     r = None if residual is None else residual.reshape(-1, w8.out_features)
     if w8.kpad != w8.in_features:
         if not w8.per_tensor:  # the quantizer writes the padding
             qa, sa = quantize_rows_padded(x2, w8.kpad)
             return gemm_i8(qa, w8.q, sa, w8.s, bias, act, residual=r).reshape(*lead, w8.out_features)
         x2 = torch.nn.functional.pad(x2, (0, w8.kpad - w8.in_features))
-    if x2.shape[0] <= 4 and pre_act == ACT_NONE and not w8.per_tensor:
-        return linear_rows(x2, w8, bias, act, r).reshape(*lead, w8.out_features)
+    if pre_act == ACT_NONE and not w8.per_tensor and (
+            x2.shape[0] <= 4 or (x2.shape[0] <= 64 and x2.is_contiguous() and x2.data_ptr() % 16 == 0)):
+        out = linear_rows(x2, w8, bias, act, r)  # both launches in one call (no tiled plan up to 64 rows)
+        return out if x.dim() == 2 else out.reshape(*lead, w8.out_features)
     qa, sa = quantize_tensor(x2) if w8.per_tensor else quantize_rows(x2, pre_act)
     out = gemm_i8(qa, w8.q, sa, w8.s, bias, act, residual=r)
     return out.reshape(*lead, w8.out_features)
@@ -767,11 +776,15 @@ def linear_rows(x2: torch.Tensor, w8: Int8Weight, bias=None, act=ACT_NONE, resid
             raise RuntimeError(f"residual shape {tuple(residual.shape)} != output {(M, N)}")
         r = residual.float().contiguous()
     out = torch.empty((M, N), dtype=torch.float32, device=x2.device)
-    need_q = want_q or M > 4 or K > 8192
-    q = torch.empty((M, K), dtype=torch.int8, device=x2.device) if need_q else None
-    s = torch.empty((M,), dtype=torch.float32, device=x2.device) if need_q else None
+    q = s = None
+    if want_q:
+        q = torch.empty((M, K), dtype=torch.int8, device=x2.device)
+        s = torch.empty((M,), dtype=torch.float32, device=x2.device)
+    elif M > 4 or K > 8192:  # the quantized rows, then their scales
+        q = torch.empty((M * (K + 4),), dtype=torch.int8, device=x2.device)
     check(lib().bq_linear_i8(x2.data_ptr(), w8.q.data_ptr(), M, N, K, w8.s.data_ptr(), _ptr(b), _ptr(r), act,
-                             out.data_ptr(), _ptr(q), _ptr(s), *_ws_args(x2.device), _stream(x2)))
+                             out.data_ptr(), _ptr(q), q.data_ptr() + M * K if s is None and q is not None else _ptr(s),
+                             *_ws_args(x2.device), _stream(x2)))
     return (out, q, s) if want_q else out
 
 
