@@ -31,22 +31,21 @@ constexpr int WA_MPW = 4;    // activation rows the per-wave kernel takes (4096 
 constexpr int WA_XLDS = 16384;       // f32 activations staged through registers (64 KB of LDS)
 constexpr int WA_XLDS_BIG = 32768;   // staged by a load loop after the weights (128 KB of LDS)
 
-// XL: the activation rows (M rows of KC * 1024 floats, K padded to whole 1 KB weight chunks)
-// are staged in LDS once per workgroup and every wave reads them from there (up to
-// WA_XLDS floats, their loads issued before the weights' and held in registers, so that
-// the wait for them is not a wait for the weights; up to WA_XLDS_BIG, by a loop after the
-// weight loads: 8 rows of 4096 at 23.8 -> 19.1 us instead of every wave reading them from
-// L2). The register staging: one row of 4096 at 7.6 -> 7.3 us, four at 12.3 -> 11.5 us.
+// The activation rows (M rows of KC * 1024 floats, K padded to whole 1 KB weight chunks) are
+// staged in LDS once per workgroup and every wave reads them from there (XN = WA_XLDS: their
+// loads issued before the weights' and held in registers, so that the wait for them is not a
+// wait for the weights; WA_XLDS_BIG, three and four rows above 4096 values: by a loop after
+// the weight loads). The register staging: one row of 4096 at 7.6 -> 7.3 us, four at 12.3 -> 11.5 us.
 // CO: the products chunk by chunk as each weight chunk lands (M = 1: one row of 4096 at
 // 7.0 -> 6.5 us); else row by row once every chunk has landed (M = 2..4: 8.0 / 9.0 / 10.1
 // us, 0.1-0.8 us less than chunk by chunk).
-template <int KC, int RPW, bool XL, int XN = WA_XLDS, bool CO = false>
+template <int KC, int RPW, int XN = WA_XLDS, bool CO = false>
 __global__ __launch_bounds__(WA_WAVES * 64) void gemv_w8a32_kernel(const float* __restrict__ x, const int8_t* W,
                                                                    int M, int N, int K, const float* __restrict__ sW,
                                                                    const float* __restrict__ bias,
                                                                    const float* __restrict__ res, int act,
                                                                    float* __restrict__ out) {
-  __shared__ __attribute__((aligned(16))) float xs[XL ? XN : 4];
+  __shared__ __attribute__((aligned(16))) float xs[XN];
   constexpr int T = WA_WAVES * 64;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -56,7 +55,7 @@ __global__ __launch_bounds__(WA_WAVES * 64) void gemv_w8a32_kernel(const float* 
   const __amdgpu_buffer_rsrc_t rw = w_rsrc(W + (size_t)min(row0, N) * K, (uint32_t)(nrows * K));
   // the activations' loads first: the wait for them (before the LDS writes) then does not
   // wait for the weight loads issued after them
-  constexpr bool XREG = XL && XN <= WA_XLDS;  // staged through registers
+  constexpr bool XREG = XN <= WA_XLDS;  // staged through registers
   constexpr int XR = XREG ? XN / 4 / T : 1;
   float4 xr[XR];
   const int k4 = K / 4;
@@ -81,31 +80,29 @@ __global__ __launch_bounds__(WA_WAVES * 64) void gemv_w8a32_kernel(const float* 
       w[j][c] = load_nt16(rw, k < K ? (uint32_t)(j * K + k) : W_OOB);
     }
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (XL) {
-    // Row m's float4 number c*256 + l*4 + t (the t-th of lane l's four in 1 KB chunk c) is
-    // stored at float4 (m*KC + c)*256 + t*64 + l, so the four reads of a chunk each take
-    // 64 consecutive float4s across the wave (no bank conflicts).
-    if constexpr (XREG) {
+  // Row m's float4 number c*256 + l*4 + t (the t-th of lane l's four in 1 KB chunk c) is
+  // stored at float4 (m*KC + c)*256 + t*64 + l, so the four reads of a chunk each take
+  // 64 consecutive float4s across the wave (no bank conflicts).
+  if constexpr (XREG) {
 #pragma unroll
-      for (int rr = 0; rr < XR; ++rr) {
-        const int i = tid + rr * T;
-        if (i < n4) {
-          const int m = i / k4;
-          const int r = i - m * k4;
-          const int dst = (m * KC + (r >> 8)) * 256 + (r & 3) * 64 + ((r >> 2) & 63);
-          reinterpret_cast<float4*>(xs)[dst] = xr[rr];
-        }
-      }
-    } else {
-      for (int i = tid; i < n4; i += T) {
+    for (int rr = 0; rr < XR; ++rr) {
+      const int i = tid + rr * T;
+      if (i < n4) {
         const int m = i / k4;
         const int r = i - m * k4;
         const int dst = (m * KC + (r >> 8)) * 256 + (r & 3) * 64 + ((r >> 2) & 63);
-        reinterpret_cast<float4*>(xs)[dst] = reinterpret_cast<const float4*>(x)[i];
+        reinterpret_cast<float4*>(xs)[dst] = xr[rr];
       }
     }
-    __syncthreads();
+  } else {
+    for (int i = tid; i < n4; i += T) {
+      const int m = i / k4;
+      const int r = i - m * k4;
+      const int dst = (m * KC + (r >> 8)) * 256 + (r & 3) * 64 + ((r >> 2) & 63);
+      reinterpret_cast<float4*>(xs)[dst] = reinterpret_cast<const float4*>(x)[i];
+    }
   }
+  __syncthreads();
   if constexpr (CO) {
     // Chunk by chunk, as the loads arrive: the chunk's effective weights f32(q) * scale, then
     // every row's FMAs against them (each output accumulates chunk by chunk, byte by byte).
@@ -127,12 +124,11 @@ __global__ __launch_bounds__(WA_WAVES * 64) void gemv_w8a32_kernel(const float* 
 #pragma unroll
       for (int m = 0; m < WA_MPW; ++m) {
         if (m >= M) break;  // uniform
-        const float4* xp = XL ? reinterpret_cast<const float4*>(xs) + (m * KC + c) * 256 + lane
-                              : reinterpret_cast<const float4*>(x + (size_t)m * K + k);
+        const float4* xp = reinterpret_cast<const float4*>(xs) + (m * KC + c) * 256 + lane;
         float xv[16];
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          const float4 v = k < K ? xp[XL ? t * 64 : t] : make_float4(0.f, 0.f, 0.f, 0.f);
+          const float4 v = k < K ? xp[t * 64] : make_float4(0.f, 0.f, 0.f, 0.f);
           xv[t * 4] = v.x; xv[t * 4 + 1] = v.y; xv[t * 4 + 2] = v.z; xv[t * 4 + 3] = v.w;
         }
 #pragma unroll
@@ -164,12 +160,11 @@ __global__ __launch_bounds__(WA_WAVES * 64) void gemv_w8a32_kernel(const float* 
       for (int c = 0; c < KC; ++c) {
         const int k = c * 1024 + lane * 16;
         if (k >= K) break;
-        const float4* xp = XL ? reinterpret_cast<const float4*>(xs) + (m * KC + c) * 256 + lane
-                              : reinterpret_cast<const float4*>(x + (size_t)m * K + k);
+        const float4* xp = reinterpret_cast<const float4*>(xs) + (m * KC + c) * 256 + lane;
         float xv[16];
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          const float4 v = xp[XL ? t * 64 : t];
+          const float4 v = xp[t * 64];
           xv[t * 4] = v.x; xv[t * 4 + 1] = v.y; xv[t * 4 + 2] = v.z; xv[t * 4 + 3] = v.w;
         }
 #pragma unroll
@@ -684,31 +679,21 @@ __global__ __launch_bounds__(256) void dequant_i8_kernel(const int8_t* __restric
   }
 }
 
-// The GEMV kernels (M <= 16, K <= 8192): the per-wave kernel below WA_MFMA_MIN_M rows, the
-// f32-MFMA one from there (its 16 MFMA columns hold up to 16 activation rows).
+// The per-wave kernel (M <= WA_MPW, K <= 8192): KC the weight chunks of a row; the activations
+// through registers where they fit (all but three and four rows above 4096 values).
 static void launch_gemv_w8a32(const float* x, const int8_t* W, int m, int n, int k, const float* sW,
                               const float* bias, const float* res, int act, float* out, hipStream_t st) {
   constexpr int RPW = 2;
   const unsigned grid = (unsigned)((n + WA_WAVES * RPW - 1) / (WA_WAVES * RPW));
-  const int64_t M = m, K = k;
-  const int64_t kc = K <= 1024 ? 1 : K <= 2048 ? 2 : K <= 4096 ? 4 : 8;  // the kernel's KC
-  if (M * kc * 1024 <= WA_XLDS) {
-    if (K <= 1024) (m == 1 ? gemv_w8a32_kernel<1, RPW, true, WA_XLDS, true> : gemv_w8a32_kernel<1, RPW, true>)<<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-    else if (K <= 2048) (m == 1 ? gemv_w8a32_kernel<2, RPW, true, WA_XLDS, true> : gemv_w8a32_kernel<2, RPW, true>)<<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-    else if (K <= 4096) (m == 1 ? gemv_w8a32_kernel<4, RPW, true, WA_XLDS, true> : gemv_w8a32_kernel<4, RPW, true>)<<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-    else (m == 1 ? gemv_w8a32_kernel<8, RPW, true, WA_XLDS, true> : gemv_w8a32_kernel<8, RPW, true>)<<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-  } else if (M * kc * 1024 <= WA_XLDS_BIG) {
-    constexpr int B = WA_XLDS_BIG;
-    if (K <= 1024) gemv_w8a32_kernel<1, RPW, true, B><<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-    else if (K <= 2048) gemv_w8a32_kernel<2, RPW, true, B><<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-    else if (K <= 4096) gemv_w8a32_kernel<4, RPW, true, B><<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-    else gemv_w8a32_kernel<8, RPW, true, B><<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-  } else {
-    if (K <= 1024) gemv_w8a32_kernel<1, RPW, false><<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-    else if (K <= 2048) gemv_w8a32_kernel<2, RPW, false><<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-    else if (K <= 4096) gemv_w8a32_kernel<4, RPW, false><<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-    else gemv_w8a32_kernel<8, RPW, false><<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
-  }
+  auto go = [&](auto kernel) {
+    kernel<<<grid, WA_WAVES * 64, 0, st>>>(x, W, m, n, k, sW, bias, res, act, out);
+  };
+  if (k <= 1024) m == 1 ? go(gemv_w8a32_kernel<1, RPW, WA_XLDS, true>) : go(gemv_w8a32_kernel<1, RPW>);
+  else if (k <= 2048) m == 1 ? go(gemv_w8a32_kernel<2, RPW, WA_XLDS, true>) : go(gemv_w8a32_kernel<2, RPW>);
+  else if (k <= 4096) m == 1 ? go(gemv_w8a32_kernel<4, RPW, WA_XLDS, true>) : go(gemv_w8a32_kernel<4, RPW>);
+  else if (m == 1) go(gemv_w8a32_kernel<8, RPW, WA_XLDS, true>);
+  else if (m == 2) go(gemv_w8a32_kernel<8, RPW>);
+  else go(gemv_w8a32_kernel<8, RPW, WA_XLDS_BIG>);
 }
 
 struct W8Ws {
