@@ -11,7 +11,7 @@
 // pieces (bq_bf16x3.h), and of the nine products of pieces the six of weight 2^-18 and above
 // are added into the f32 accumulator, smallest first. The three left out are below 2^-26 of
 // the product, under the f32 rounding of the sum; measured against float64 on N(0, 1) inputs
-// the output's relative error is 2.5e-7, where f32 MFMAs gave 3.3e-7.
+// the output's relative error is 2.7e-7, where f32 MFMAs gave 3.3e-7.
 //
 // k's planes are staged in LDS once, split there by the whole workgroup, and v's take their
 // place after the scores: 80 KB at 208 keys, so that two workgroups share a CU and one's loads
@@ -24,7 +24,8 @@
 // a 32-key step takes keys 32 s + 16 (e / 4) + 4 g + e % 4 as group g's eight, and row n of block
 // d is head dim 4 n + d, so that v is written to LDS and the output to memory in whole pieces.
 //
-// ViT-B/16 at 32 images (197 tokens, 12 heads): 70 -> 38.5 us; 256 tokens 88 -> 59 us (98 KB of LDS, one workgroup a CU).
+// ViT-B/16 at 32 images (197 tokens, 12 heads): 69.5 -> 34.5 us; 256 tokens 88 -> 59 us (98 KB
+// of LDS, one workgroup a CU).
 #include <math.h>
 
 #include "bq_bf16x3.h"
