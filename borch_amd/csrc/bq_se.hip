@@ -87,213 +87,124 @@ __global__ __launch_bounds__(SE_THREADS) void se_partial_kernel(const float* __r
   }
 }
 
-// 16 bytes of a buffer, zeros past its end (SE_OOB and up), without a branch a load.
-constexpr uint32_t SE_OOB = 0x80000000u;
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t se_rsrc(const float* base, size_t floats) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, (int)(floats * 4), 0x00020000);
-}
-__device__ __forceinline__ float4 se_load(__amdgpu_buffer_rsrc_t r, bool in, int float4s) {
-  return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, in ? (uint32_t)float4s * 16u : SE_OOB, 0, 0));
-}
-__device__ __forceinline__ float4 add4(float4 a, float4 b) {
-  return make_float4(__fadd_rn(a.x, b.x), __fadd_rn(a.y, b.y), __fadd_rn(a.z, b.z), __fadd_rn(a.w, b.w));
-}
-__device__ __forceinline__ float4 max4(float4 a, float4 b) {
-  return make_float4(fmaxf(a.x, b.x), fmaxf(a.y, b.y), fmaxf(a.z, b.z), fmaxf(a.w, b.w));
-}
-__device__ __forceinline__ float4 fma4(float a, float4 b, float4 c) {
-  return make_float4(__fmaf_rn(a, b.x, c.x), __fmaf_rn(a, b.y, c.y), __fmaf_rn(a, b.z, c.z), __fmaf_rn(a, b.w, c.w));
-}
-
 // One block per image: pooled and max |x| per channel (in LDS), z = silu(W1 pooled + b1)
-// (one wave per output j, its lanes over c, a wave tree), gate = sigmoid(W2 z + b2) from the
-// transposed expand weight w2t [S, C]. With `amax`: max over c of fl(max|x[n, :, c]| *
-// gate[n, c]) into amax[n]. (Splitting the squeeze and the excite into two wider kernels was
-// slower on every B0 layer: each small launch pays its own latency chain.)
-//
-// The chain of memory round trips bounds it, at most a block an image being in flight. So the
-// weights come as 16-byte loads, all that a thread needs of a layer at once (up to 15 of w1,
-// issued before the pooled sums they wait for, and 16 of w2t, before the barrier on z). More
-// than 4 chunks or 16 terms are split over up to R row lanes a channel group of 4 (thread t:
-// group t % G, row lane t / G), which meet through LDS in lane order; fewer are not, a meeting
-// costing what a round trip does. Loads that no lane needs are skipped: out of range they cost
-// the address unit as much (1.5-2.5 us at C <= 480).
-// A call's two kernels at 32 images: C = 1152 at 7x7 19.6 -> 15.0 us, 672 at 14x14 15.2 -> 12.9,
-// 480 11.5 -> 10.2, C <= 240 the same (144 at 28x28, whose 6 chunks meet, 8.7 -> 9.6), against
-// 4-byte loads in batches of 20 and 32 and one thread a channel.
+// (one wave per output j, its lanes over c, a wave tree), gate = sigmoid(W2 z + b2) (one
+// thread per channel, reading the transposed expand weight w2t [S, C] so a wave's loads are
+// contiguous). With `amax`: max over c of fl(max|x[n, :, c]| * gate[n, c]) into amax[n].
+// (Splitting the squeeze and the excite into two wider kernels was slower on every B0
+// layer: 9-18 us against 5.5-18 us, each small launch paying its own latency chain.)
 __global__ __launch_bounds__(GATE_THREADS) void se_gate_kernel(const float* __restrict__ partial,
                                                              const float* __restrict__ pmax, int chunks, int HW,
-                                                             int C, int S, int R, const float* __restrict__ w1,
+                                                             int C, int S, const float* __restrict__ w1,
                                                              const float* __restrict__ b1,
                                                              const float* __restrict__ w2t,
                                                              const float* __restrict__ b2, float* __restrict__ gate,
                                                              float* __restrict__ amax) {
-  extern __shared__ __attribute__((aligned(16))) float sm[];  // pooled [C], xmax [C], red [R > 1: 2][R][C], z [S]
+  extern __shared__ float sm[];  // pooled [C], z [S], xmax [C] (with amax)
   __shared__ float wmax[GATE_THREADS / 64];
-  constexpr int WAVES = GATE_THREADS / 64;
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-  const int G = C / 4, GW = min(G, GATE_THREADS);
-  float4* const pooled = reinterpret_cast<float4*>(sm);
-  float4* const xmax = pooled + G;
-  float4* const red = xmax + G;  // R > 1 only (then G <= GATE_THREADS / 2: one pass over the groups)
-  float* const z = sm + 2 * C + (R > 1 ? 2 * R * C : 0);
-  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int rl = t / GW, g0 = t - rl * GW;
+  float* pooled = sm;
+  float* z = sm + C;
+  float* xmax = sm + C + S;
   const int n = blockIdx.x;
   const float inv = __fdiv_rn(1.0f, (float)HW);
-
-  constexpr int JW = 3, CU = 5;
-  const __amdgpu_buffer_rsrc_t r1 = se_rsrc(w1, (size_t)S * C);
-  float4 wv[JW][CU];
-  auto load_w1 = [&](int jb, int cb) {  // outputs jb + 16 q, channel groups cb + 64 u
+  for (int c = threadIdx.x; c < C; c += GATE_THREADS) {
+    float s = 0.f, m = 0.f;
+    for (int k0 = 0; k0 < chunks; k0 += 8) {  // eight loads in flight, added in chunk order
+      float v[8], w[8];
 #pragma unroll
-    for (int q = 0; q < JW; ++q)
-#pragma unroll
-      for (int u = 0; u < CU; ++u) {
-        const int j = jb + WAVES * q, c4 = cb + 64 * u;
-        wv[q][u] = zero;
-        if (j < S && cb - lane + 64 * u < G) wv[q][u] = se_load(r1, c4 < G, j * G + c4);  // uniform
-      }
-  };
-  load_w1(wave, lane);
-  __builtin_amdgcn_sched_barrier(0);
-
-  const int KL = min(R, (chunks + 3) / 4);  // row lanes that the chunks need
-  const size_t image = (size_t)n * chunks * C;
-  const __amdgpu_buffer_rsrc_t rs = se_rsrc(partial + image, (size_t)chunks * C);
-  const __amdgpu_buffer_rsrc_t rm = se_rsrc(amax ? pmax + image : partial, amax ? (size_t)chunks * C : 0);
-  for (int gb = 0; gb < G; gb += GW) {
-    const int g = gb + g0;
-    const bool mine = rl < KL && g < G;
-    float4 s = zero, m = zero;
-    for (int kb = 0; mine && kb < chunks; kb += 4 * KL) {  // four chunks' loads in flight, added in order
-      float4 v[4], w[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int k = kb + rl + u * KL;
-        v[u] = w[u] = zero;
-        if (kb + u * KL < chunks) {  // uniform
-          v[u] = se_load(rs, k < chunks, k * G + g);
-          w[u] = se_load(rm, k < chunks, k * G + g);
-        }
+      for (int k = 0; k < 8; ++k) {
+        const size_t o = ((size_t)n * chunks + k0 + k) * C + c;
+        v[k] = k0 + k < chunks ? partial[o] : 0.f;
+        w[k] = (amax && k0 + k < chunks) ? pmax[o] : 0.f;
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        s = add4(s, v[u]);
-        m = max4(m, w[u]);
+      for (int k = 0; k < 8; ++k) {
+        if (k0 + k < chunks) s = __fadd_rn(s, v[k]);
+        m = fmaxf(m, w[k]);
       }
     }
-    if (KL > 1) {  // uniform
-      if (mine) {
-        red[rl * G + g] = s;
-        red[(R + rl) * G + g] = m;
-      }
-      __syncthreads();
-      if (mine && rl == 0)
-        for (int k = 1; k < KL; ++k) {
-          s = add4(s, red[k * G + g]);
-          m = max4(m, red[(R + k) * G + g]);
-        }
-    }
-    if (mine && rl == 0) {
-      pooled[g] = make_float4(__fmul_rn(s.x, inv), __fmul_rn(s.y, inv), __fmul_rn(s.z, inv), __fmul_rn(s.w, inv));
-      xmax[g] = m;
-    }
+    pooled[c] = __fmul_rn(s, inv);
+    if (amax) xmax[c] = m;
   }
   __syncthreads();
-
-  // z: lane l of a wave takes channel groups l, l + 64, ... in order, then a fixed-order wave sum
-  for (int jb = wave; jb < S; jb += WAVES * JW) {
+  // z: each wave builds JW outputs at once, its lanes over c (c = lane, lane + 64, ... in
+  // order for every output), all loads of a batch issued before its FMAs; then a fixed-order
+  // DPP wave sum.
+  constexpr int JW = 4, CU = 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int j0 = wave * JW; j0 < S; j0 += (GATE_THREADS / 64) * JW) {
     float acc[JW];
 #pragma unroll
     for (int q = 0; q < JW; ++q) acc[q] = 0.f;
-    for (int cb = lane; cb - lane < G; cb += 64 * CU) {
-      if (jb != wave || cb != lane) load_w1(jb, cb);
+    for (int c0 = lane; c0 < C; c0 += 64 * CU) {
+      float pv[CU], wv[JW][CU];
 #pragma unroll
       for (int u = 0; u < CU; ++u) {
-        if (cb - lane + 64 * u >= G) break;  // uniform
-        const float4 pv = cb + 64 * u < G ? pooled[cb + 64 * u] : zero;
+        const int c = c0 + 64 * u;
+        pv[u] = c < C ? pooled[c] : 0.f;
 #pragma unroll
-        for (int q = 0; q < JW; ++q) {
-          const float4 w = wv[q][u];
-          acc[q] = __fmaf_rn(w.w, pv.w, __fmaf_rn(w.z, pv.z, __fmaf_rn(w.y, pv.y, __fmaf_rn(w.x, pv.x, acc[q]))));
-        }
+        for (int q = 0; q < JW; ++q) wv[q][u] = (c < C && j0 + q < S) ? w1[(size_t)(j0 + q) * C + c] : 0.f;
       }
+#pragma unroll
+      for (int u = 0; u < CU; ++u)
+#pragma unroll
+        for (int q = 0; q < JW; ++q) acc[q] = __fmaf_rn(wv[q][u], pv[u], acc[q]);
     }
 #pragma unroll
     for (int q = 0; q < JW; ++q) {
-      const int j = jb + WAVES * q;
       const float v = wave_sum_fixed(acc[q]);  // the whole wave is here (the loop is per wave)
-      if (lane == 0 && j < S) z[j] = silu(__fadd_rn(v, b1 ? b1[j] : 0.f));
+      if (lane == 0 && j0 + q < S) z[j0 + q] = silu(__fadd_rn(v, b1 ? b1[j0 + q] : 0.f));
     }
   }
-
-  constexpr int JU = 16;
-  const int JL = min(R, (S + JU - 1) / JU);  // row lanes that the terms need
-  const __amdgpu_buffer_rsrc_t r2 = se_rsrc(w2t, (size_t)S * C);
-  float4 ev[JU];
-  auto load_w2 = [&](int jb, int g) {  // terms jb + rl + JL v
-#pragma unroll
-    for (int v = 0; v < JU; ++v) {
-      const int j = jb + rl + JL * v;
-      ev[v] = zero;
-      if (jb + JL * v < S) ev[v] = se_load(r2, j < S, j * G + g);  // uniform
-    }
-  };
-  if (rl < JL) load_w2(0, g0);
-  __builtin_amdgcn_sched_barrier(0);
   __syncthreads();
-  float peak = 0.f;
-  for (int gb = 0; gb < G; gb += GW) {
-    const int g = gb + g0;
-    const bool mine = rl < JL && g < G;
-    float4 acc = zero;
-    for (int jb = 0; mine && jb < S; jb += JL * JU) {
-      if (jb || gb) load_w2(jb, g);
+  // gate: each thread CW channels at once (c0, c0 + 1024, ...), j in order, JU loads of w2t
+  // a channel issued before their FMAs.
+  constexpr int CW = 4, JU = 8;
+  float m = 0.f;
+  for (int c0 = threadIdx.x; c0 < C; c0 += GATE_THREADS * CW) {
+    float acc[CW];
+#pragma unroll
+    for (int u = 0; u < CW; ++u) {
+      const int c = c0 + GATE_THREADS * u;
+      acc[u] = (b2 && c < C) ? b2[c] : 0.f;
+    }
+    for (int j0 = 0; j0 < S; j0 += JU) {
+      float wv[JU][CW], zv[JU];
 #pragma unroll
       for (int v = 0; v < JU; ++v) {
-        const int j = jb + rl + JL * v;
-        if (jb + JL * v < S) acc = fma4(j < S ? z[j] : 0.f, ev[v], acc);
-      }
-    }
-    if (JL > 1) {  // uniform
-      if (mine) red[rl * G + g] = acc;
-      __syncthreads();
-      if (mine && rl == 0)
-        for (int k = 1; k < JL; ++k) acc = add4(acc, red[k * G + g]);
-    }
-    if (mine && rl == 0) {
-      const float a[4] = {acc.x, acc.y, acc.z, acc.w};
-      const float4 x4 = xmax[g];
-      const float xm[4] = {x4.x, x4.y, x4.z, x4.w};
+        zv[v] = j0 + v < S ? z[j0 + v] : 0.f;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int c = 4 * g + e;
-        const float y = sigmoid_f(b2 ? __fadd_rn(a[e], b2[c]) : a[e]);
-        gate[(size_t)n * C + c] = y;
-        peak = fmaxf(peak, __fmul_rn(xm[e], y));
+        for (int u = 0; u < CW; ++u) {
+          const int c = c0 + GATE_THREADS * u;
+          wv[v][u] = (j0 + v < S && c < C) ? w2t[(size_t)(j0 + v) * C + c] : 0.f;
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < JU; ++v)
+#pragma unroll
+        for (int u = 0; u < CW; ++u) acc[u] = __fmaf_rn(wv[v][u], zv[v], acc[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < CW; ++u) {
+      const int c = c0 + GATE_THREADS * u;
+      if (c < C) {
+        const float g = sigmoid_f(acc[u]);
+        gate[(size_t)n * C + c] = g;
+        if (amax) m = fmaxf(m, __fmul_rn(xmax[c], g));
       }
     }
   }
   if (amax) {  // uniform
-    peak = wave_max(peak);
-    if (lane == 0) wmax[wave] = peak;
+    m = wave_max(m);
+    if (lane == 0) wmax[wave] = m;
     __syncthreads();
-    if (t == 0) {
+    if (threadIdx.x == 0) {
       float r = wmax[0];
 #pragma unroll
-      for (int w = 1; w < WAVES; ++w) r = fmaxf(r, wmax[w]);
+      for (int w = 1; w < GATE_THREADS / 64; ++w) r = fmaxf(r, wmax[w]);
       amax[n] = r;
     }
   }
-}
-
-// Row lanes a channel group: the threads over the groups, at most 16 (each adds an LDS read to
-// the meeting), one where their sums would not fit beside the rest in 64 KB of LDS.
-static size_t gate_lds(int64_t C, int64_t S, int R) { return (size_t)(2 * C + S + (R > 1 ? 2 * R * C : 0)) * sizeof(float); }
-static int gate_lanes(int64_t C, int64_t S) {
-  const int R = (int)std::min<int64_t>(GATE_THREADS / std::min<int64_t>(C / 4, GATE_THREADS), 16);
-  return gate_lds(C, S, R) + 1024 <= 64 * 1024 ? R : 1;
 }
 
 static int se_chunks(int64_t HW, int64_t C) {
@@ -390,9 +301,9 @@ int bq_se_gate_nhwc(const float* x, int64_t N, int64_t HW, int64_t C, const floa
   se_partial_kernel<<<(unsigned)(N * chunks), SE_THREADS, 0, st>>>(x, (int)HW, (int)C, chunks, rows_per, partial,
                                                                    absmax_parts ? pmax : nullptr);
   if (int r = check_launch(what)) return r;
-  const int R = gate_lanes(C, S);
-  se_gate_kernel<<<(unsigned)N, GATE_THREADS, gate_lds(C, S, R), st>>>(partial, pmax, chunks, (int)HW, (int)C, (int)S, R,
-                                                                       w1, b1, w2t, b2, gate, absmax_parts);
+  const size_t lds = (size_t)(C + S + (absmax_parts ? C : 0)) * sizeof(float);
+  se_gate_kernel<<<(unsigned)N, GATE_THREADS, lds, st>>>(partial, pmax, chunks, (int)HW, (int)C, (int)S, w1, b1, w2t,
+                                                         b2, gate, absmax_parts);
   return check_launch(what);
 }
 
