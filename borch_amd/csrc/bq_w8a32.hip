@@ -705,7 +705,7 @@ static void launch_w8a32_ksplit(const W8P& p, const W8Ws& ws, hipStream_t st) {
   const int tiles = ((p.M + 16 * FM - 1) / (16 * FM)) * ((p.N + 16 * FN - 1) / (16 * FN));
   const int KT = (p.K + 63) / 64;
   int S = std::max(1, std::min(256 / tiles, KT / W8_WAVES));
-  const int per = (KT + S - 1) / S;
+  const int per = std::max(1, (KT + S - 1) / S);  // K = 0 has one empty slice
   S = (KT + per - 1) / per;  // no empty slice
   if ((size_t)tiles * S * FM * FN * 1024 > W8_WS_BYTES - W8_CNT_BYTES || tiles * 4 > (int)W8_CNT_BYTES) S = 1;
   const bool split = S > 1 && ws.ptr && ws.bytes >= W8_WS_BYTES;
