@@ -309,25 +309,37 @@ struct W8P {
   int vec;           // N % 4 == 0 and every pointer 16-byte aligned: whole float4s
 };
 
-// The plain f32 sum of one output. The split leaves NaN where x is infinite or rounds to a
-// bf16 infinity, so a sum that is not finite is taken again this way: an infinity, a NaN or
-// an overflow of the f32 sum itself then comes out as f32 arithmetic gives it.
-__device__ __attribute__((noinline)) float w8_dot_f32(const float* x, const int8_t* w, int K) {
+// The f32 sum of one output over the effective weights, as the kernels for fewer rows take it.
+__device__ __attribute__((noinline)) float w8_dot_f32(const float* x, const int8_t* w, float sc, int K) {
   float s = 0.f;
-  for (int k = 0; k < K; ++k) s = __fmaf_rn(x[k], (float)w[k], s);
+  for (int k = 0; k < K; ++k) s = __fmaf_rn(x[k], __fmul_rn((float)w[k], sc), s);
   return s;
 }
 
-// Outputs n .. n + 3 of row m from their sums.
+// Outputs n .. n + 3 of row m from their sums. An output whose scaled sum is not finite is taken
+// again over the effective weights f32(q) * s: the split leaves NaN where x is infinite or rounds
+// to a bf16 infinity, the sum of x * q can overflow where that of x * (q * s) does not (x = 3e36,
+// q = 127, s = 1 / 127), and an infinite scale makes NaN of a zero weight. So an infinity, a NaN
+// or an overflow comes out as f32 arithmetic on the effective weights gives it.
 __device__ __forceinline__ void w8_store4(const W8P& p, int m, int n, v4f v) {
   if (m >= p.M || n >= p.N) return;
+  float s[4];
+  if (p.vec) {
+    const float4 s4 = *reinterpret_cast<const float4*>(p.sW + n);
+    s[0] = s4.x; s[1] = s4.y; s[2] = s4.z; s[3] = s4.w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] = n + e < p.N ? p.sW[n + e] : 0.f;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = __fmul_rn(v[e], s[e]);
   if (!__builtin_isfinite(v[0] + v[1] + v[2] + v[3]))
-    for (int e = 0; e < 4 && n + e < p.N; ++e)
-      v[e] = w8_dot_f32(p.x + (size_t)m * p.K, p.W + (size_t)(n + e) * p.K, p.K);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < p.N) v[e] = w8_dot_f32(p.x + (size_t)m * p.K, p.W + (size_t)(n + e) * p.K, s[e], p.K);
   const size_t o = (size_t)m * p.N + n;
   if (p.vec) {
-    const float4 s = *reinterpret_cast<const float4*>(p.sW + n);
-    float4 y = make_float4(__fmul_rn(v[0], s.x), __fmul_rn(v[1], s.y), __fmul_rn(v[2], s.z), __fmul_rn(v[3], s.w));
+    float4 y = make_float4(v[0], v[1], v[2], v[3]);
     if (p.bias) {
       const float4 b = *reinterpret_cast<const float4*>(p.bias + n);
       y = make_float4(__fadd_rn(y.x, b.x), __fadd_rn(y.y, b.y), __fadd_rn(y.z, b.z), __fadd_rn(y.w, b.w));
@@ -342,7 +354,7 @@ __device__ __forceinline__ void w8_store4(const W8P& p, int m, int n, v4f v) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       if (n + e >= p.N) return;
-      float y = __fmul_rn(v[e], p.sW[n + e]);
+      float y = v[e];
       if (p.bias) y = __fadd_rn(y, p.bias[n + e]);
       if (p.res) y = __fadd_rn(y, p.res[o + e]);
       p.out[o + e] = activate(y, p.act);

@@ -438,7 +438,8 @@ int bq_se_gate_nhwc(const float* x, int64_t N, int64_t HW, int64_t C, const floa
  * FMA accumulation, as the reference; M <= 16 over a short K: the same weights on the f32 MFMA.
  * Otherwise bf16-MFMA kernels: q is exact in bf16 and each x is split exactly into three bf16
  * pieces, so every product is exact; the f32 accumulation is the only rounding before
- * y = fl(sum * sW[n]) (a sum that comes out infinite or NaN is taken again in plain f32). Either way
+ * y = fl(sum * sW[n]) (a y that comes out infinite or NaN is taken again in f32 over the effective
+ * weights, so an infinity, a NaN or an overflow is what those give). Either way
  * every output is within (K + 2) 2^-24 sum_k |x * w| + 2^-24 |y| of the exact result on the
  * effective weights w = f32(q) * sW. The int8 weight is read inside the kernel: no f32 copy
  * of it is written. K % 16 == 0; x and W 16-byte aligned; x and W each < 2 GiB.

@@ -1,4 +1,5 @@
-"""The weight-only Linear at the ends of its size range, in every kernel: empty products."""
+"""The weight-only Linear at the ends of its value and size ranges, in every kernel: empty products,
+sums that overflow before their scale, infinite scales."""
 from __future__ import annotations
 
 import pytest
@@ -8,6 +9,13 @@ pytestmark = pytest.mark.gpu
 
 from borch_amd import int8 as I  # noqa: E402
 from borch_amd._lib import check, lib  # noqa: E402
+
+INF = float("inf")
+
+
+def _packed(q, s):
+    return I.Int8Weight(q.to(torch.int8).contiguous(), s.contiguous(), q.shape[1], q.shape[0], True)
+
 
 @pytest.mark.parametrize("M,N", [(3, 40), (8, 17), (40, 300), (600, 4099)])
 def test_empty_product(M, N):
@@ -20,3 +28,49 @@ def test_empty_product(M, N):
     check(lib().bq_linear_w8a32(pad.data_ptr(), pad.data_ptr(), M, N, 0, b.data_ptr(), b.data_ptr(), r.data_ptr(),
                                 I.ACT_RELU, out.data_ptr(), st))
     assert torch.equal(out, torch.relu(b + r))
+
+
+# rows of the f32-MFMA kernel, the K-split one's forms and the tiled one's
+SHAPES = [(4, 64, 1024), (8, 64, 1024), (6, 300, 4096), (16, 4096, 4112), (16, 2048, 8208), (20, 768, 3072),
+          (40, 2051, 2064), (256, 3072, 1040), (600, 4099, 144), (1700, 2051, 144)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_sums_that_overflow_before_their_scale(M, N, K):
+    """x * q sums past f32's range while x * (q * s) stays in it: finite, as the effective weights'
+    products give it. Every third row is of ordinary size."""
+    print(f"w8a32 large x M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device="cuda")
+    q = torch.randint(-127, 128, (N, K), generator=g, device="cuda")
+    s = (0.5 + torch.rand(N, generator=g, device="cuda")) / 127
+    big = torch.arange(M, device="cuda") % 3 != 0
+    x[big, 0] = 3.0e36
+    q[:, 0] = 127 - torch.arange(N, device="cuda") % 40  # x * q is past 2.6e38, or near it, from the first value on
+    x[big, 1:] *= 1e30
+    w8 = _packed(q, s)
+    y = I.linear_w8a32(x, w8)
+    wd = q.double() * s.double()[:, None]
+    want = x.double() @ wd.t()
+    assert bool(torch.isfinite(y).all())
+    mag = x.double().abs() @ wd.abs().t()
+    assert bool(((y.double() - want).abs() <= (K + 3) * 2.0 ** -24 * mag + 2.0 ** -23 * want.abs()).all())
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_infinite_scale(M, N, K):
+    """f32(0) * inf is NaN in the effective weight, so a channel with an infinite scale is NaN where
+    any of its weights is 0, and an infinity of the sum's sign, or NaN, elsewhere."""
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.rand(M, K, generator=g, device="cuda") + 0.5
+    q = torch.randint(1, 128, (N, K), generator=g, device="cuda")
+    s = torch.full((N,), 0.01, device="cuda")
+    s[0], s[N // 2], s[N - 1] = INF, INF, INF
+    q[0, 3] = 0
+    q[N // 2, 5] = -1
+    y = I.linear_w8a32(x, _packed(q, s))
+    assert bool(torch.isnan(y[:, 0]).all()) and bool(torch.isnan(y[:, N // 2]).all())  # 0 * inf; inf - inf
+    assert bool((y[:, N - 1] == INF).all())
+    rest = torch.ones(N, dtype=torch.bool, device="cuda")
+    rest[[0, N // 2, N - 1]] = False
+    assert bool(torch.isfinite(y[:, rest]).all())

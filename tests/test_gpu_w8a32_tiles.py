@@ -99,8 +99,6 @@ def test_non_finite_rows(M):
         ok = ~torch.isnan(want)
         assert torch.equal(y[r][ok].double(), want[ok])
     sums = (xi[3].double() @ q.t())
-    safe = sums.abs() < 3e38  # the f32 sum stays finite
-    want = (sums * w8.s.double() + b.double())
-    assert bool(safe.any())
-    assert torch.allclose(y[3][safe].double(), want[safe], rtol=1e-5)
+    want = (sums * w8.s.double() + b.double())  # finite, also where the sum before its scale is not
+    assert torch.allclose(y[3].double(), want, rtol=1e-5)
     assert torch.equal(y[5:], plain[5:])
