@@ -98,6 +98,7 @@ __global__ __launch_bounds__(T) void quantize_rows_kernel(const float* __restric
 // torch pad before it took two kernels more for (1000 x 1555: 13.7 us as fill, copy and
 // quantize_rows_kernel). Rows in registers up to NV * 4 * T values; NV == 0 reads them twice.
 typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));
+constexpr int64_t PAD_KMAX = 0x7ffff000;  // a row's last index and a thread's next step after it fit an int
 
 __device__ __forceinline__ float4 row4(const float* xr, int k, int K) {
   if (k + 3 < K) {
@@ -653,7 +654,7 @@ int bq_quantize_rows_padded(const float* x, int64_t M, int64_t K, int64_t Kp, in
   if (M < 0 || K < 0 || Kp < K) return set_error(BQ_ERR_ARG, "%s: bad sizes M=%lld K=%lld Kp=%lld", what, (long long)M, (long long)K, (long long)Kp);
   if (M == 0) return BQ_OK;
   if ((!x && K > 0) || !q || !s) return set_error(BQ_ERR_ARG, "%s: null pointer", what);
-  if (M > 0x7fffffff || Kp > 0x7ffffff0) return set_error(BQ_ERR_ARG, "%s: size too large", what);
+  if (M > 0x7fffffff || Kp > PAD_KMAX) return set_error(BQ_ERR_ARG, "%s: size too large", what);
   if (Kp % 4 || ((uintptr_t)q & 3) || ((uintptr_t)x & 3))
     return set_error(BQ_ERR_UNSUPPORTED, "%s: Kp %% 4 == 0 and 4-byte aligned x and q", what);
   auto go = [&](auto kernel, int threads) {
@@ -674,7 +675,7 @@ int bq_pad_rows_f32(const float* x, int64_t M, int64_t K, int64_t Kp, float* y, 
   if (M < 0 || K < 0 || Kp < K) return set_error(BQ_ERR_ARG, "%s: bad sizes M=%lld K=%lld Kp=%lld", what, (long long)M, (long long)K, (long long)Kp);
   if (M == 0 || Kp == 0) return BQ_OK;
   if ((!x && K > 0) || !y) return set_error(BQ_ERR_ARG, "%s: null pointer", what);
-  if (Kp > 0x7ffffff0) return set_error(BQ_ERR_ARG, "%s: size too large", what);
+  if (Kp > PAD_KMAX) return set_error(BQ_ERR_ARG, "%s: size too large", what);
   if (Kp % 4 || ((uintptr_t)y & 15) || ((uintptr_t)x & 3))
     return set_error(BQ_ERR_UNSUPPORTED, "%s: Kp %% 4 == 0, y 16-byte and x 4-byte aligned", what);
   const dim3 grid((unsigned)((Kp / 4 + 255) / 256), (unsigned)(M < 65535 ? M : 65535));

@@ -79,13 +79,13 @@ int bq_quantize_rows_act(const float* x, int64_t M, int64_t K, int act, int8_t* 
                          bq_stream_t stream);
 
 /* bq_quantize_rows of rows whose width is no multiple of a vector: x f32 [M, K] at 4-byte
- * alignment -> q int8 [M, Kp], zeros from K on (Kp >= K, Kp % 4 == 0; q 4-byte aligned), s f32
+ * alignment -> q int8 [M, Kp], zeros from K on (K <= Kp <= 2^31 - 4096, Kp % 4 == 0; q 4-byte aligned), s f32
  * [M]: the same bytes and scales. The zero padding of the reference's packed rows (quant.ts:42-51)
  * without a padded copy of x. */
 int bq_quantize_rows_padded(const float* x, int64_t M, int64_t K, int64_t Kp, int8_t* q, float* s,
                             bq_stream_t stream);
 
-/* x f32 [M, K] at 4-byte alignment -> y f32 [M, Kp], zeros from K on (Kp % 4 == 0; y 16-byte
+/* x f32 [M, K] at 4-byte alignment -> y f32 [M, Kp], zeros from K on (Kp as above; y 16-byte
  * aligned): the activations of a weight-only Linear padded to its packed weight's width. */
 int bq_pad_rows_f32(const float* x, int64_t M, int64_t K, int64_t Kp, float* y, bq_stream_t stream);
 
