@@ -53,16 +53,18 @@ def capture(fn, calls):
     """A HIP graph of ``calls`` back-to-back ``fn(i)`` launches (no host launch cost on
     replay: the sub-10 us kernels would otherwise be timed at the Python call rate)."""
     import torch
+    from borch_amd import int8 as I
     s = torch.cuda.Stream()
     s.wait_stream(torch.cuda.current_stream())
-    with torch.cuda.stream(s):
-        for i in range(calls):
-            fn(i)
-    torch.cuda.current_stream().wait_stream(s)
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g, stream=s):  # the warm-up stream: its split-K workspace is recorded
-        for i in range(calls):
-            fn(i)
+    with I.graph_workspaces({}) as g.workspaces:  # kept with the graph, which records them
+        with torch.cuda.stream(s):
+            for i in range(calls):
+                fn(i)
+        torch.cuda.current_stream().wait_stream(s)
+        with torch.cuda.graph(g, stream=s):  # the stream the warm-up made them for
+            for i in range(calls):
+                fn(i)
     return g
 
 

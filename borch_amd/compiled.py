@@ -13,7 +13,7 @@ the same input shape overwrites it (clone it to keep it).
 
 Split (``split=n``, graph mode): the batch runs as ``n`` chunks on parallel streams inside
 the one graph, so one chunk's store- or latency-bound kernels overlap another's MFMA work
-(each stream with its own split-K workspace). Refused where it would change the result:
+(each stream with its own split-K workspace, all of them the graph's). Refused where it would change the result:
 a conv with a dynamic per-tensor input scale takes the maximum over the whole batch, so the
 model needs calibrated scales (``calibrate_int8``) or per-row (Linear) quantization only.
 Measured at n = 2: EfficientNet-B0 b64 calibrated 1.55 -> 1.41 ms, ViT-B/16 b32 3.09 ->
@@ -48,7 +48,7 @@ class Compiled:
         self.split = int(split)
         if self.split < 1:
             raise ValueError(f"split must be >= 1, got {split}")
-        self._streams = {}  # device -> [stream], made on its first split call (each with its own split-K workspace)
+        self._streams = {}  # device -> [stream], made on its first split call
         self.tuned = []  # the tuner's decisions, one list per input shape (borch_amd.tune.tune)
         self._tuned_keys = set()
         self.int8_layers = 0
@@ -79,10 +79,10 @@ class Compiled:
         if not self._split_ok(x):
             return self.model(x)
         streams = self._streams.get(x.device)
-        if streams is None:  # the warm-up runs come first, outside any capture
+        if streams is None:
             streams = self._streams[x.device] = [torch.cuda.Stream(device=x.device) for _ in range(self.split)]
-            for s in streams:  # each chunk stream's split-K workspace, made now (outside any capture)
-                _i8.split_workspace(x.device, s)
+        for s in streams:  # each chunk stream's split-K workspace, made by the warm-up runs (outside any capture)
+            _i8.split_workspace(x.device, s)
         cur = torch.cuda.current_stream(x.device)
         outs = []
         for s, xc in zip(streams, x.chunk(self.split)):
@@ -107,19 +107,26 @@ class Compiled:
             static_in = x.clone()
             s = torch.cuda.Stream(device=x.device)
             s.wait_stream(torch.cuda.current_stream(x.device))
-            with torch.cuda.stream(s):
-                for _ in range(2):  # warm up the allocator and any lazy init outside capture
-                    self._run(static_in)
-            torch.cuda.current_stream(x.device).wait_stream(s)
-            g = torch.cuda.CUDAGraph()
-            # captured on the warm-up stream: the split-K workspace made for it is the one
-            # the graph records
-            with torch.cuda.graph(g, stream=s):
-                static_out = self._run(static_in)
-            entry = (g, static_in, static_out)
+            # the graph's own split-K workspaces, made by the warm-up on the stream that is then
+            # captured: torch hands out its streams again, and graphs captured on one stream may
+            # be replayed on two at once
+            with _i8.graph_workspaces({}) as workspaces:
+                with torch.cuda.stream(s):
+                    for _ in range(2):  # warm up the allocator and any lazy init outside capture
+                        self._run(static_in)
+                torch.cuda.current_stream(x.device).wait_stream(s)
+                g = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(g, stream=s):
+                    static_out = self._run(static_in)
+            entry = (g, static_in, static_out, workspaces, set())
             self._graphs[key] = entry
-        g, static_in, static_out = entry
+        g, static_in, static_out, workspaces, replayed_on = entry
         static_in.copy_(x)
+        cur = torch._C._cuda_getCurrentRawStream(x.device.index)
+        if cur not in replayed_on:  # the workspaces go with this object, but not before its replays there have run
+            replayed_on.add(cur)
+            for ws in workspaces.values():
+                ws.record_stream(torch.cuda.current_stream(x.device))
         g.replay()
         return static_out
 

@@ -8,7 +8,9 @@ its conv input). There is no CPU path: a tensor that is not on a gfx950 device r
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import threading
 from dataclasses import dataclass
 
 import torch
@@ -24,6 +26,7 @@ __all__ = [
     "pack_linear_weight", "pack_conv_weight", "attention_f32", "avgpool_linear",
     "quantize_nhwc_scaled", "quantize_nhwc_chscale", "se_gate_nhwc", "linear_w8a32", "dequant_weight",
     "pack_dw_weight", "linear", "linear_rows", "conv2d", "depthwise_conv2d", "round_up", "split_workspace",
+    "graph_workspaces",
 ]
 
 
@@ -48,34 +51,79 @@ def _stream(t: torch.Tensor):
 # each have their own tile counters and partials. (torch hands out streams from a fixed
 # pool per device, so the table stays small.)
 _SPLIT_WS: dict = {}
+# The same for the eager calls of the weight-only Linear, which no graph records: two calls on
+# different streams never share one, whatever has been captured on either.
+_W8A32_WS: dict = {}
+
+
+class _Owned(threading.local):
+    table = None  # the workspaces of the graph this thread is making (graph_workspaces)
+
+
+_OWNED = _Owned()
+
+
+@contextlib.contextmanager
+def graph_workspaces(table: dict):
+    """Calls of this thread inside the block take their split-K workspaces from ``table``
+    (``{}`` at first; made on a call outside any capture). Warm up and capture a graph in one
+    such block and keep ``table`` as long as the graph: its workspaces are then its own, and
+    it may run beside any other graph or call, where graphs captured on one stream would
+    share that stream's. A replay on another stream: ``record_stream`` them there."""
+    before, _OWNED.table = _OWNED.table, table
+    try:
+        yield table
+    finally:
+        _OWNED.table = before
 
 
 def split_workspace(device: torch.device, stream=None):
     """The split-K workspace of ``stream`` (default: the current stream) on ``device``, or
     None while a graph is being captured on a stream that has none yet (those calls then
     run unsplit: the same results). Capture on the stream the warm-up ran on to keep it."""
+    return _workspace(_SPLIT_WS if _OWNED.table is None else _OWNED.table, device, stream)
+
+
+def _workspace(table: dict, device: torch.device, stream=None):
     idx = torch.device(device).index
     idx = torch.cuda.current_device() if idx is None else idx
     st = torch.cuda.current_stream(idx) if stream is None else stream
     key = (idx, st.cuda_stream)
-    ws = _SPLIT_WS.get(key)
+    ws = table.get(key)
     if ws is None:
         if torch.cuda.is_current_stream_capturing():
             return None
-        with torch.cuda.stream(st):
+        # a graph's own goes back to the allocator with the graph, so it comes from the default
+        # stream's memory, where the next graph finds it (a capture's stream is hardly ever the same)
+        at = st if table is not _OWNED.table else torch.cuda.default_stream(idx)
+        with torch.cuda.stream(at):
             ws = torch.zeros(int(lib().bq_gemm_ws_bytes()), dtype=torch.uint8, device=torch.device("cuda", idx))
-        _SPLIT_WS[key] = ws
+        if at is not st:
+            st.wait_stream(at)
+            ws.record_stream(st)
+        table[key] = ws
     return ws
 
 
-def _ws_args(device):
-    """(pointer, bytes) of the current stream's split-K workspace, or (None, 0) (unsplit)."""
+def _ws_args(device, shared=_SPLIT_WS):
+    """(pointer, bytes) of the current stream's split-K workspace (the graph's being made, else
+    ``shared``'s), or (None, 0) (unsplit)."""
+    table = shared if _OWNED.table is None else _OWNED.table
     ws = None
     if device.index is not None:  # one that is there already
-        ws = _SPLIT_WS.get((device.index, torch._C._cuda_getCurrentRawStream(device.index)))
+        ws = table.get((device.index, torch._C._cuda_getCurrentRawStream(device.index)))
     if ws is None:
-        ws = split_workspace(device)
+        ws = _workspace(table, device)
     return (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
+
+
+def _w8a32_ws_args(device):
+    """``_ws_args`` of the weight-only Linear. A capture that does not own its workspaces gets
+    none (the slices in turn, the same bits): the stream's would be shared with every other
+    graph captured there and with the eager calls on it."""
+    if _OWNED.table is None and torch.cuda.is_current_stream_capturing():
+        return None, 0
+    return _ws_args(device, _W8A32_WS)
 
 
 def _need(t: torch.Tensor, name: str, dtype: torch.dtype) -> None:
@@ -389,8 +437,9 @@ def linear_w8a32(x: torch.Tensor, w8: Int8Weight, bias=None, act=ACT_NONE, resid
         if tuple(residual.shape[:-1]) != tuple(lead) or residual.shape[-1] != N:
             raise RuntimeError(f"residual shape {tuple(residual.shape)} != output {(*lead, N)}")
         r = residual.reshape(M, N).float().contiguous()
+    ws = (None, 0) if M <= 4 and K <= 8192 else _w8a32_ws_args(x2.device)  # the GEMV splits nothing
     check(lib().bq_linear_w8a32_ws(x2.data_ptr(), w8.q.data_ptr(), M, N, K, w8.s.data_ptr(), _ptr(b), _ptr(r), act,
-                                   out.data_ptr(), *_ws_args(x2.device), _stream(x2)))
+                                   out.data_ptr(), *ws, _stream(x2)))
     return out.reshape(*lead, N)
 
 
@@ -777,14 +826,16 @@ def linear_rows(x2: torch.Tensor, w8: Int8Weight, bias=None, act=ACT_NONE, resid
         r = residual.float().contiguous()
     out = torch.empty((M, N), dtype=torch.float32, device=x2.device)
     q = s = None
+    gemv = M <= 4 and K <= 8192  # one launch: nothing quantized in memory, nothing split
     if want_q:
         q = torch.empty((M, K), dtype=torch.int8, device=x2.device)
         s = torch.empty((M,), dtype=torch.float32, device=x2.device)
-    elif M > 4 or K > 8192:  # the quantized rows, then their scales
+    elif not gemv:  # the quantized rows, then their scales
         q = torch.empty((M * (K + 4),), dtype=torch.int8, device=x2.device)
+    ws = (None, 0) if gemv else _ws_args(x2.device)
     check(lib().bq_linear_i8(x2.data_ptr(), w8.q.data_ptr(), M, N, K, w8.s.data_ptr(), _ptr(b), _ptr(r), act,
                              out.data_ptr(), _ptr(q), q.data_ptr() + M * K if s is None and q is not None else _ptr(s),
-                             *_ws_args(x2.device), _stream(x2)))
+                             *ws, _stream(x2)))
     return (out, q, s) if want_q else out
 
 
