@@ -309,56 +309,114 @@ struct W8P {
   int vec;           // N % 4 == 0 and every pointer 16-byte aligned: whole float4s
 };
 
-// The f32 sum of one output over the effective weights, as the kernels for fewer rows take it.
-__device__ __attribute__((noinline)) float w8_dot_f32(const float* x, const int8_t* w, float sc, int K) {
-  float s = 0.f;
-  for (int k = 0; k < K; ++k) s = __fmaf_rn(x[k], __fmul_rn((float)w[k], sc), s);
-  return s;
+// Outputs of one row that a wave takes again over the effective weights f32(q) * s: lane l's
+// n .. n + 3 for the lanes of `again`, 64 lanes a sum (in a fixed order). Lanes l, l + 16, l + 32 and
+// l + 48 hold the same row m; `row` is what is known of it from an earlier call (0 nothing, 1 no
+// NaN, 2 a NaN). A NaN in x decides its whole row, so a row is searched for one first, and only
+// rows without pay for sums: a batch that has gone NaN costs one more read of x (256 x 4096 x 4096
+// 0.044 ms -> 0.09, where a lane summed each output alone 7.5), an infinity in every row the sums
+// (6304 x 768 x 3072 0.11 -> 2.4 ms, 34 so).
+struct W8Again {
+  v4f y;
+  int row;
+};
+__device__ __attribute__((noinline)) W8Again w8_again(const float* x, const int8_t* W, int N, int K, int m, int n, v4f y,
+                                                      v4f s, int row, uint64_t again) {
+  const int lane = threadIdx.x & 63;
+  for (int r = 0; r < 16; ++r) {  // uniform, as every test below but the last of each row
+    uint64_t todo = again & (0x0001000100010001ull << r);
+    if (!todo) continue;
+    const float* xr = x + (size_t)__shfl(m, __builtin_ffsll((long long)todo) - 1) * K;
+    int known = __shfl(row, r);
+    if (known == 0) {
+      bool nan = false;
+      for (int k = lane * 4; k < K; k += 256) {
+        const float4 v = *reinterpret_cast<const float4*>(xr + k);
+        nan = nan || __builtin_isnan(v.x) || __builtin_isnan(v.y) || __builtin_isnan(v.z) || __builtin_isnan(v.w);
+      }
+      known = __ballot(nan) ? 2 : 1;
+    }
+    if ((lane & 15) == r) row = known;
+    for (; todo; todo &= todo - 1) {
+      const int l = __builtin_ffsll((long long)todo) - 1;
+      const int nl = __shfl(n, l);
+      float a[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] = known == 2 ? __builtin_nanf("") : 0.f;
+      if (known != 2) {
+        float sc[4];
+        const int8_t* w[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          sc[e] = __shfl(s[e], l);
+          w[e] = W + (size_t)min(nl + e, N - 1) * K;
+        }
+        for (int k = lane * 4; k < K; k += 256) {
+          const float4 v = *reinterpret_cast<const float4*>(xr + k);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const uint32_t q = *reinterpret_cast<const uint32_t*>(w[e] + k);
+            a[e] = __fmaf_rn(v.x, __fmul_rn((float)(int8_t)(q & 0xff), sc[e]), a[e]);
+            a[e] = __fmaf_rn(v.y, __fmul_rn((float)(int8_t)((q >> 8) & 0xff), sc[e]), a[e]);
+            a[e] = __fmaf_rn(v.z, __fmul_rn((float)(int8_t)((q >> 16) & 0xff), sc[e]), a[e]);
+            a[e] = __fmaf_rn(v.w, __fmul_rn((float)(int8_t)(q >> 24), sc[e]), a[e]);
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] = wave_sum_fixed(a[e]);
+      }
+      if (lane == l) y = (v4f){a[0], a[1], a[2], a[3]};
+    }
+  }
+  return W8Again{y, row};
 }
 
-// Outputs n .. n + 3 of row m from their sums. An output whose scaled sum is not finite is taken
-// again over the effective weights f32(q) * s: the split leaves NaN where x is infinite or rounds
-// to a bf16 infinity, the sum of x * q can overflow where that of x * (q * s) does not (x = 3e36,
-// q = 127, s = 1 / 127), and an infinite scale makes NaN of a zero weight. So an infinity, a NaN
-// or an overflow comes out as f32 arithmetic on the effective weights gives it.
-__device__ __forceinline__ void w8_store4(const W8P& p, int m, int n, v4f v) {
-  if (m >= p.M || n >= p.N) return;
-  float s[4];
-  if (p.vec) {
-    const float4 s4 = *reinterpret_cast<const float4*>(p.sW + n);
-    s[0] = s4.x; s[1] = s4.y; s[2] = s4.z; s[3] = s4.w;
-  } else {
+// Outputs n .. n + 3 of row m from their sums; the whole wave calls it. An output whose scaled
+// sum is not finite is taken again over the effective weights f32(q) * s: the split leaves NaN
+// where x is infinite or rounds to a bf16 infinity, the sum of x * q can overflow where that of
+// x * (q * s) does not (x = 3e36, q = 127, s = 1 / 127), and an infinite scale makes NaN of a zero
+// weight. So an infinity, a NaN or an overflow comes out as f32 arithmetic on the effective
+// weights gives it. `row`: w8_again's, 0 where the lane's row is another than in the last call.
+__device__ __forceinline__ void w8_store4(const W8P& p, int m, int n, v4f v, int& row) {
+  const bool in = m < p.M && n < p.N;
+  const size_t o = (size_t)m * p.N + n;
+  v4f s = {0.f, 0.f, 0.f, 0.f}, bias = s, res = s;  // loaded together, before the test that needs the scales
+  if (in) {
+    if (p.vec) {
+      s = *reinterpret_cast<const v4f*>(p.sW + n);
+      if (p.bias) bias = *reinterpret_cast<const v4f*>(p.bias + n);
+      if (p.res) res = *reinterpret_cast<const v4f*>(p.res + o);
+    } else {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s[e] = n + e < p.N ? p.sW[n + e] : 0.f;
+      for (int e = 0; e < 4; ++e)
+        if (n + e < p.N) {
+          s[e] = p.sW[n + e];
+          if (p.bias) bias[e] = p.bias[n + e];
+          if (p.res) res[e] = p.res[o + e];
+        }
+    }
   }
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = __fmul_rn(v[e], s[e]);
-  if (!__builtin_isfinite(v[0] + v[1] + v[2] + v[3]))
+  const uint64_t again = __ballot(in && !__builtin_isfinite(v[0] + v[1] + v[2] + v[3]));
+  if (again) {
+    const W8Again a = w8_again(p.x, p.W, p.N, p.K, m, n, v, s, row, again);
+    v = a.y;
+    row = a.row;
+  }
+  if (!in) return;
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (n + e < p.N) v[e] = w8_dot_f32(p.x + (size_t)m * p.K, p.W + (size_t)(n + e) * p.K, s[e], p.K);
-  const size_t o = (size_t)m * p.N + n;
+  for (int e = 0; e < 4; ++e) {
+    if (p.bias) v[e] = __fadd_rn(v[e], bias[e]);
+    if (p.res) v[e] = __fadd_rn(v[e], res[e]);
+    v[e] = activate(v[e], p.act);
+  }
   if (p.vec) {
-    float4 y = make_float4(v[0], v[1], v[2], v[3]);
-    if (p.bias) {
-      const float4 b = *reinterpret_cast<const float4*>(p.bias + n);
-      y = make_float4(__fadd_rn(y.x, b.x), __fadd_rn(y.y, b.y), __fadd_rn(y.z, b.z), __fadd_rn(y.w, b.w));
-    }
-    if (p.res) {
-      const float4 r = *reinterpret_cast<const float4*>(p.res + o);
-      y = make_float4(__fadd_rn(y.x, r.x), __fadd_rn(y.y, r.y), __fadd_rn(y.z, r.z), __fadd_rn(y.w, r.w));
-    }
-    *reinterpret_cast<float4*>(p.out + o) =
-        make_float4(activate(y.x, p.act), activate(y.y, p.act), activate(y.z, p.act), activate(y.w, p.act));
+    *reinterpret_cast<v4f*>(p.out + o) = v;
   } else {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (n + e >= p.N) return;
-      float y = v[e];
-      if (p.bias) y = __fadd_rn(y, p.bias[n + e]);
-      if (p.res) y = __fadd_rn(y, p.res[o + e]);
-      p.out[o + e] = activate(y, p.act);
-    }
+    for (int e = 0; e < 4; ++e)
+      if (n + e < p.N) p.out[o + e] = v[e];
   }
 }
 
@@ -547,7 +605,8 @@ __global__ __launch_bounds__(W8_WAVES * 64) void w8a32_ksplit_kernel(W8P p, int 
   for (int u = 0; u < PER; ++u) {
     const int e = tid + u * T;
     const int l = e & 63, j = (e >> 6) % FN, i = (e >> 6) / FN;
-    if (ITEMS % T == 0 || e < ITEMS) w8_store4(p, m0 + 16 * i + (l & 15), n0 + 16 * j + 4 * (l >> 4), sum[u]);
+    int row = 0;
+    if (ITEMS % T == 0 || e < ITEMS) w8_store4(p, m0 + 16 * i + (l & 15), n0 + 16 * j + 4 * (l >> 4), sum[u], row);
   }
 }
 
@@ -669,9 +728,11 @@ __global__ __launch_bounds__(WAVES * 64, 4) void w8a32_tile_kernel(W8P p) {
     if (c + 1 < KT) chunk(c + 1, 1);
   }
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+  for (int i = 0; i < FM; ++i) {
+    int row = 0;
 #pragma unroll
-    for (int j = 0; j < FN; ++j) w8_store4(p, m0 + 16 * i + r, n0 + 16 * j + 4 * g, acc[i][j]);
+    for (int j = 0; j < FN; ++j) w8_store4(p, m0 + 16 * i + r, n0 + 16 * j + 4 * g, acc[i][j], row);
+  }
 }
 
 // w[n, k] = f32(q[n, k]) * s[n] (one rounding), four elements a thread.

@@ -74,3 +74,54 @@ def test_infinite_scale(M, N, K):
     rest = torch.ones(N, dtype=torch.bool, device="cuda")
     rest[[0, N // 2, N - 1]] = False
     assert bool(torch.isfinite(y[:, rest]).all())
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_non_finite_values(M, N, K):
+    """Rows with one infinity, two of either sign, a NaN, only NaN, beside finite ones: NaN and
+    infinity where float64 on the effective weights has them, the other rows' bits unchanged."""
+    print(f"w8a32 non-finite M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device="cuda")
+    w8 = I.pack_linear_weight(torch.randn(N, K, generator=g, device="cuda"), weight_only=True)
+    b = torch.randn(N, generator=g, device="cuda")
+    plain = I.linear_w8a32(x, w8, b)
+    xi = x.clone()
+    at = torch.arange(M, device="cuda") % 7
+    if M < 7:
+        at[:4] = torch.arange(4, device="cuda")
+    xi[at == 0, K - 1] = INF
+    xi[at == 1, 2] = -INF
+    xi[at == 1, K // 2] = INF
+    xi[at == 2, K // 3] = float("nan")
+    xi[at == 3] = float("nan")
+    y = I.linear_w8a32(xi, w8, b)
+    wd = (w8.q.double() * w8.s.double()[:, None]).t().contiguous()
+    bad = at < 4
+    want = xi[bad].double() @ wd + b.double()
+    assert torch.equal(torch.isnan(y[bad]), torch.isnan(want))
+    inf = torch.isinf(want)
+    assert bool(inf.any()) and torch.equal(y[bad][inf].double(), want[inf])
+    assert torch.equal(y[~bad], plain[~bad])
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 1024, 4096), (2048, 2048, 512)])
+def test_a_batch_of_nan_costs_little_more(M, N, K):
+    """A NaN in x decides its row, so its outputs need no second sum: such a batch takes about
+    twice the time of a finite one (30 times when each output was summed again)."""
+    w8 = I.pack_linear_weight(torch.randn(N, K, device="cuda"), weight_only=True)
+
+    def us(x):
+        best = 1e9
+        for _ in range(8):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(8):
+                I.linear_w8a32(x, w8)
+            e1.record()
+            e1.synchronize()
+            best = min(best, e0.elapsed_time(e1) * 125)
+        return best
+    x = torch.randn(M, K, device="cuda")
+    t = us(x), us(torch.full_like(x, float("nan")))
+    assert t[1] < 6 * t[0] + 20, t
