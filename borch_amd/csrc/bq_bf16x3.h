@@ -3,10 +3,11 @@
 // x = x1 + x2 + x3 with x1 the bf16 nearest x and x2 the bf16 nearest x - x1: x - x1 is a
 // multiple of ulp_f32(x) below 2^-8 |x| (at most 16 significant bits), (x - x1) - x2 a
 // multiple of it below 2^-16 |x| (at most 8), so x3 = (x - x1) - x2 is exact in bf16 and the
-// split loses nothing (|x| >= 2^-109, so that no piece falls below bf16's last bit; smaller
-// values lose at most 2^-134 in absolute terms; the MFMA takes bf16 subnormals as they are).
-// Just below 2^128 x1 may round to infinity, and an infinite x leaves NaN in x2, so either
-// makes every sum it is part of NaN or infinite: callers take such sums again in plain f32.
+// split loses nothing for |x| >= 2^-109. Below that pieces fall under bf16's last bit, 2^-133 (the
+// MFMA takes bf16 subnormals as they are), and a value loses up to 2^-134. Just below 2^128 x1
+// may round to infinity, and an infinite x leaves NaN in x2, so either makes every sum it is part
+// of NaN or infinite. Callers take sums again in plain f32 that are not finite or so small that
+// such a loss matters.
 #pragma once
 
 #include "bq_common.h"

@@ -376,7 +376,9 @@ __device__ __attribute__((noinline)) W8Again w8_again(const float* x, const int8
 // where x is infinite or rounds to a bf16 infinity, the sum of x * q can overflow where that of
 // x * (q * s) does not (x = 3e36, q = 127, s = 1 / 127), and an infinite scale makes NaN of a zero
 // weight. So an infinity, a NaN or an overflow comes out as f32 arithmetic on the effective
-// weights gives it. `row`: w8_again's, 0 where the lane's row is another than in the last call.
+// weights gives it. So is a sum below K * 2^-103, zero aside: values below 2^-109 lose up to 2^-134
+// in the split, so a larger sum at most 127 K 2^-134 < 2^-24 of itself. `row`: w8_again's, 0 where
+// the lane's row is another than in the last call.
 __device__ __forceinline__ void w8_store4(const W8P& p, int m, int n, v4f v, int& row) {
   const bool in = m < p.M && n < p.N;
   const size_t o = (size_t)m * p.N + n;
@@ -396,9 +398,14 @@ __device__ __forceinline__ void w8_store4(const W8P& p, int m, int n, v4f v, int
         }
     }
   }
+  uint32_t least = ~0u;  // |sum| as an integer, 0 as the largest
 #pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = __fmul_rn(v[e], s[e]);
-  const uint64_t again = __ballot(in && !__builtin_isfinite(v[0] + v[1] + v[2] + v[3]));
+  for (int e = 0; e < 4; ++e) {
+    least = min(least, (__float_as_uint(v[e]) & 0x7fffffffu) - 1u);
+    v[e] = __fmul_rn(v[e], s[e]);
+  }
+  const bool lost = least < __float_as_uint((float)p.K * 0x1p-103f) - 1u;
+  const uint64_t again = __ballot(in && (lost || !__builtin_isfinite(v[0] + v[1] + v[2] + v[3])));
   if (again) {
     const W8Again a = w8_again(p.x, p.W, p.N, p.K, m, n, v, s, row, again);
     v = a.y;

@@ -125,3 +125,34 @@ def test_a_batch_of_nan_costs_little_more(M, N, K):
     x = torch.randn(M, K, device="cuda")
     t = us(x), us(torch.full_like(x, float("nan")))
     assert t[1] < 6 * t[0] + 20, t
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -100, 2.0 ** -112, 2.0 ** -118, 2.0 ** -124])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_tiny_values(M, N, K, scale):
+    """Activations whose bf16 pieces fall below bf16's last bit, in rows of their own (scales of up
+    to 2^30 keep the outputs normal numbers), beside ordinary rows and rows of zeros: within the f32
+    accumulation's bound, and no bit of the others changed."""
+    print(f"w8a32 tiny M={M} N={N} K={K} scale={scale}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device="cuda")
+    q = torch.randint(-127, 128, (N, K), generator=g, device="cuda")
+    q[1] = 0  # an empty output channel
+    s = torch.exp2(30 * torch.rand(N, generator=g, device="cuda"))
+    w8 = _packed(q, s)
+    plain = I.linear_w8a32(x, w8)
+    rows = torch.arange(M, device="cuda") % 3
+    x[rows == 1] *= scale
+    x[rows == 2] = 0
+    y = I.linear_w8a32(x, w8)
+    wd = (q.double() * s.double()[:, None]).t().contiguous()
+    tiny = x[rows == 1].double()
+    want, mag = tiny @ wd, tiny.abs() @ wd.abs()
+    # an f32 sum over the effective weights or scaled after it (one more rounding), and underflow:
+    # half of f32's last bit, 2^-150, a product and sum
+    bound = (K + 3) * 2.0 ** -24 * mag + 2.0 ** -23 * want.abs() + 2 * K * 2.0 ** -150
+    err = (y[rows == 1].double() - want).abs()
+    assert bool((err <= bound).all()), float((err / bound).max())
+    # and as a whole as close as ordinary values come (about 4e-7): the lost bits are 2^-17 of 2^-118
+    assert float(err.norm() / want.norm()) < 2e-6
+    assert torch.equal(y[rows == 0], plain[rows == 0]) and not bool(y[rows == 2].any())
