@@ -40,7 +40,8 @@ __device__ __forceinline__ float xor_max(float v, int m) { return fmaxf(v, __shf
 __device__ __forceinline__ float xor_add(float v, int m) { return __fadd_rn(v, __shfl_xor(v, m)); }
 
 // Attention of query q of one head by one wave in plain f32: for queries whose outputs did not
-// come out finite above (an infinity among the inputs, or a value a bf16 piece cannot hold).
+// come out finite above (an infinity among the inputs, or a value a bf16 piece cannot hold) or
+// came out smaller than the pieces of v reach.
 // Lane l scores keys l, l + 64, ..., then sums head dim l.
 __device__ __attribute__((noinline)) void attention_f32_query(const float* base, size_t tok, int T, int D, int q,
                                                               float* orow) {
@@ -258,14 +259,21 @@ __global__ __launch_bounds__(ATT_WAVES * 64, KB <= 13 ? 4 : 2) void attention_f3
   }
   float* orow = out + ((size_t)b * T + q) * D + (size_t)h * ATT_DH;
   float4 y[4];
-  bool finite = true;
+  // taken again: an output that is not finite, or (zero aside) below 2^-109, where the up to 2^-134
+  // that the split takes from a smaller v is more than a rounding
+  float zero = 0.f;  // NaN beside a value that is not finite
+  uint32_t least = ~0u;  // |y| as an integer, 0 as the largest
+  auto look = [&](float v) {
+    zero = __fmaf_rn(v, 0.f, zero);
+    least = min(least, (__float_as_uint(v) << 1) - 1u);
+  };
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     y[r] = make_float4(__fdiv_rn(o[0][r], sum), __fdiv_rn(o[1][r], sum), __fdiv_rn(o[2][r], sum), __fdiv_rn(o[3][r], sum));
-    finite = finite && __builtin_isfinite(y[r].x) && __builtin_isfinite(y[r].y) && __builtin_isfinite(y[r].z) &&
-             __builtin_isfinite(y[r].w);
+    look(y[r].x); look(y[r].y); look(y[r].z); look(y[r].w);
   }
-  uint64_t again = __ballot(q < T && !finite);  // bit n of each 16: query q0 + n
+  const bool good = zero == 0.f && least >= (__float_as_uint(0x1p-109f) << 1) - 1u;
+  uint64_t again = __ballot(q < T && !good);  // bit n of each 16: query q0 + n
   again |= again >> 32;
   again |= again >> 16;
   if (q < T && !((again >> n) & 1))

@@ -438,12 +438,14 @@ int bq_se_gate_nhwc(const float* x, int64_t N, int64_t HW, int64_t C, const floa
  * FMA accumulation, as the reference; M <= 16 over a short K: the same weights on the f32 MFMA.
  * Otherwise bf16-MFMA kernels: q is exact in bf16 and each x is split exactly into three bf16
  * pieces (|x| >= 2^-109; below, up to 2^-134 a value is lost), so every product is exact; the f32
- * accumulation is the only rounding before y = fl(sum * sW[n]) (a y that comes out infinite or NaN,
- * or so small that the lost bits matter, is taken again in f32 over the effective weights, so an infinity, a NaN or an overflow is what those give; the time of such a call
- * depends on its data: rows of x with a NaN cost little, one with an infinity N more sums). Either way
- * every output is within (K + 2) 2^-24 sum_k |x * w| + 2^-24 |y| (and underflow: 2^-150 a product,
- * 2^-127 sW a value of x below 2^-133) of the exact result on the effective weights w = f32(q) * sW. The int8 weight is read inside the kernel: no f32 copy
- * of it is written. K % 16 == 0; x and W 16-byte aligned; x and W each < 2 GiB.
+ * accumulation is the only rounding before y = fl(sum * sW[n]). A y that comes out infinite or
+ * NaN, or so small that the lost bits matter, is taken again in f32 over the effective weights, so
+ * an infinity, a NaN or an overflow is what those give; the time of such a call depends on its
+ * data (a row of x with a NaN costs little, one with an infinity N more sums). Either way every
+ * output is within (K + 2) 2^-24 sum_k |x * w| + 2^-24 |y| (and underflow: 2^-150 a product,
+ * 2^-127 sW a value of x below 2^-133) of the exact result on the effective weights
+ * w = f32(q) * sW. The int8 weight is read inside the kernel: no f32 copy of it is written.
+ * K % 16 == 0; x and W 16-byte aligned; x and W each < 2 GiB.
  * Replaces matmul(..., weightInt8) (borch-ts/src/kernels.ts:2661-2753, the int8 read at
  * 2695-2708) and its routing (tensor.ts:2553-2575) for streamed / windowed weights
  * (Tensor.inWindowInt8, tensor.ts:1681-1705; stream_sequential(int8=True),
