@@ -442,26 +442,27 @@ __device__ __forceinline__ v4i w8_transpose(v4i w) {
 // Few rows: a workgroup owns 16 FM x 16 FN outputs over one of S slices of K, and its waves
 // split the slice (wave w takes chunks w, w + WAVES, ...), each straight from memory into
 // registers, PF chunks ahead; the waves' partial blocks meet through LDS in wave order, the
-// slices' through the workspace in slice order (`part` null: this workgroup takes every slice
-// in turn, which gives the same sums). As in the int8 GEMM's K split, no workgroup waits for
+// slices' through the workspace in slice order (TURNS, without a workspace: this workgroup takes
+// every slice in turn, which gives the same sums). As in the int8 GEMM's K split, no workgroup waits for
 // another: a tile's last one (its counter) adds the slices, runs the epilogue and clears the
 // counter; partials are device-scope relaxed atomics, complete before the counter's increment.
 //
 // What bounds it is the bytes a CU pulls through its L1, x above all (four bytes a value
 // against the weight's one): 16 rows of 4096 are 256 KB in every workgroup of a grid that only
 // splits N. Slices of K cut that, for the 2-3 us that the exchange of partials takes: 16 rows
-// against a 4096 x 4096 weight 13.5 us unsliced, 11.6 us as 64 tiles of 16 x 64 in 4 slices
-// (f32 MFMA on the unsplit rows, as below but for this K: 15.5 us). Against 32 x 64 tiles
-// staged through LDS: M = 17 35.8 -> 13.1 us, M = 64 36.2 -> 19.9, M = 256 47.8 -> 41.0.
-template <int FM, int FN, int PF>
-__global__ __launch_bounds__(W8_WAVES * 64) void w8a32_ksplit_kernel(W8P p, int S, int* cnt, uint64_t* part) {
-  constexpr int WAVES = W8_WAVES, T = WAVES * 64, ITEMS = FM * FN * 64, PER = (ITEMS + T - 1) / T;
-  __shared__ __attribute__((aligned(16))) v4f red[WAVES * ITEMS];
+// against a 4096 x 4096 weight 13.5 us unsliced, 11.1 us as 64 tiles of 16 x 64 in 4 slices
+// (f32 MFMA on the unsplit rows, as below but for this K: 15.4 us). Against 32 x 64 tiles
+// staged through LDS: M = 17 35.8 -> 13.0 us, M = 64 36.0 -> 19.0, M = 256 44.7 -> 36.8.
+template <int FM, int FN, int PF, bool TURNS, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void w8a32_ksplit_kernel(W8P p, int S, int* cnt, uint64_t* part) {
+  constexpr int T = WAVES * 64, ITEMS = FM * FN * 64, PER = (ITEMS + T - 1) / T;
+  constexpr int G = TURNS ? (FM * FN == 1 ? 8 : 2) : 1;  // slices whose blocks meet at a time
+  __shared__ __attribute__((aligned(16))) v4f red[G * WAVES * ITEMS];
   __shared__ int s_last;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, g = lane >> 4;
   const int K = p.K;
-  const int groups = part ? S : 1;  // workgroups of a tile
+  const int groups = TURNS ? 1 : S;  // workgroups of a tile
   const int id = xcd_order(blockIdx.x, gridDim.x);
   const int tiles_m = (p.M + 16 * FM - 1) / (16 * FM), tiles_n = (p.N + 16 * FN - 1) / (16 * FN);
   int bm, bn;
@@ -495,15 +496,105 @@ __global__ __launch_bounds__(W8_WAVES * 64) void w8a32_ksplit_kernel(W8P p, int 
     const uint32_t off = c * 64 + 16 * g < K ? wo[j] + c * 64 : W_OOB;
     wb[s][j] = FM == 1 ? load_nt16(rw, off) : __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, off, 0, 0));
   };
-  const int KT = (K + 63) / 64, per = (KT + S - 1) / S;
-  v4f sum[PER];
-  for (int q = 0; q < S / groups; ++q) {
-    const int c_begin = (slice + q) * per, c_end = min(KT, c_begin + per);
-    v4f acc[FM][FN];
+  v4f acc[FM][FN];
+  auto clear = [&]() {
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int j = 0; j < FN; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
+  };
+  // A chunk's products, its registers taking chunk `next` (`more`: there is one) as they fall free.
+  auto products = [&](int s, bool more, int next) __attribute__((always_inline)) {
+    Split8 a[2][FM];  // x is split first
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < FM; ++i) a[h][i] = split8(xb[s][i][2 * h], xb[s][i][2 * h + 1]);
+    if (more) {
+      load_x(s, next);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const v4i w = w8_transpose(wb[s][j]);
+      if (more) load_w(s, j, next);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const v8bf b = i8x8_bf16((uint32_t)w[2 * h], (uint32_t)w[2 * h + 1]);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[h][i].p3, acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[h][i].p2, acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[h][i].p1, acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  auto put = [&](int at) {  // this wave's blocks, as those of slice `at` of the G
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) red[(((at * WAVES + wave) * FM + i) * FN + j) * 64 + lane] = acc[i][j];
+  };
+  v4f sum[PER];
+  auto meet = [&](int n, bool first) {  // n slices' blocks, the waves of each in order
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int e = tid + u * T;
+      if (ITEMS % T == 0 || e < ITEMS)
+        for (int at = 0; at < n; ++at) {
+          const v4f* from = red + at * WAVES * ITEMS + e;
+          v4f v = from[0];
+#pragma unroll
+          for (int w = 1; w < WAVES; ++w) v += from[w * ITEMS];
+          sum[u] = first && at == 0 ? v : sum[u] + v;
+        }
+    }
+  };
+  const int KT = (K + 63) / 64, per = (KT + S - 1) / S;
+  clear();
+  if constexpr (TURNS) {
+    // every slice in this workgroup, the loads running on from one slice into the next; all waves
+    // have chunks in every slice but, maybe, the last (slices hold at least a chunk a wave)
+    int q = 0, c = wave, nq = 0, nc = wave;  // the chunk at hand and the next one to load
+    auto forth = [&](int& sl, int& ch) {
+      ch += WAVES;
+      if (ch >= min(KT, (sl + 1) * per)) ch = ++sl * per + wave;
+    };
+    const auto valid = [&](int sl, int ch) { return sl < S && ch < min(KT, (sl + 1) * per); };
+#pragma unroll
+    for (int s = 0; s < PF; ++s) {
+      if (!valid(nq, nc)) break;  // uniform across the wave, as below
+#pragma unroll
+      for (int j = 0; j < FN; ++j) load_w(s, j, nc);
+      load_x(s, nc);
+      forth(nq, nc);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    while (valid(q, c)) {
+#pragma unroll
+      for (int s = 0; s < PF; ++s) {
+        if (!valid(q, c)) break;
+        products(s, valid(nq, nc), nc);
+        if (valid(nq, nc)) forth(nq, nc);
+        const int was = q;
+        forth(q, c);
+        if (q != was && q < S) {  // slice `was` is done and another follows
+          put(was % G);
+          clear();
+          if (was % G == G - 1) {
+            __syncthreads();
+            meet(G, was < G);
+            __syncthreads();
+          }
+        }
+      }
+    }
+    put((S - 1) % G);
+    __syncthreads();
+    meet((S - 1) % G + 1, S <= G);
+  } else {
+    const int c_begin = slice * per, c_end = min(KT, c_begin + per);
 #pragma unroll
     for (int s = 0; s < PF; ++s) {
       const int c = c_begin + wave + s * WAVES;
@@ -518,48 +609,12 @@ __global__ __launch_bounds__(W8_WAVES * 64) void w8a32_ksplit_kernel(W8P p, int 
       for (int s = 0; s < PF; ++s) {
         const int c = c0 + s * WAVES, next = c + WAVES * PF;
         if (c >= c_end) break;
-        Split8 a[2][FM];  // x is split first: its registers then take the chunk PF ahead
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int i = 0; i < FM; ++i) a[h][i] = split8(xb[s][i][2 * h], xb[s][i][2 * h + 1]);
-        if (next < c_end) {
-          load_x(s, next);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          const v4i w = w8_transpose(wb[s][j]);
-          if (next < c_end) load_w(s, j, next);
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const v8bf b = i8x8_bf16((uint32_t)w[2 * h], (uint32_t)w[2 * h + 1]);
-#pragma unroll
-            for (int i = 0; i < FM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[h][i].p3, acc[i][j], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < FM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[h][i].p2, acc[i][j], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < FM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[h][i].p1, acc[i][j], 0, 0, 0);
-          }
-        }
+        products(s, next < c_end, next);
       }
     }
-    if (q) __syncthreads();  // the previous slice's blocks have been read
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j) red[((wave * FM + i) * FN + j) * 64 + lane] = acc[i][j];
+    put(0);
     __syncthreads();
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int e = tid + u * T;
-      if (ITEMS % T == 0 || e < ITEMS) {
-        v4f v = red[e];
-#pragma unroll
-        for (int w = 1; w < WAVES; ++w) v += red[w * ITEMS + e];
-        sum[u] = q ? sum[u] + v : v;
-      }
-    }
+    meet(1, true);
   }
   if (groups > 1) {
     const int tile = bm * tiles_n + bn;
@@ -780,18 +835,39 @@ struct W8Ws {
   void* ptr;
   size_t bytes;
 };
+// Slices of K of an output block of 16 fm rows: up to 256 workgroups, each slice at least a chunk a wave.
+static int w8a32_slices(const W8P& p, int fm, int fn) {
+  const int64_t tiles = (int64_t)((p.M + 16 * fm - 1) / (16 * fm)) * ((p.N + 16 * fn - 1) / (16 * fn));
+  const int KT = (p.K + 63) / 64;
+  int S = std::max(1, std::min((int)(256 / tiles), KT / W8_WAVES));
+  const int per = std::max(1, (KT + S - 1) / S);  // K = 0 has one empty slice
+  S = std::max(1, (KT + per - 1) / per);  // no empty slice
+  const bool fits = (size_t)tiles * S * fm * fn * 1024 <= W8_WS_BYTES - W8_CNT_BYTES && tiles * 4 <= (int64_t)W8_CNT_BYTES;
+  return fits ? S : 1;
+}
+template <int FM, int FN, int PF, bool TURNS = false, int WAVES = W8_WAVES>
+static void launch_w8a32_blocks(const W8P& p, int S, const W8Ws& ws, hipStream_t st) {
+  const unsigned tiles = (unsigned)(((p.M + 16 * FM - 1) / (16 * FM)) * ((p.N + 16 * FN - 1) / (16 * FN)));
+  const bool split = !TURNS && S > 1;
+  w8a32_ksplit_kernel<FM, FN, PF, TURNS, WAVES><<<split ? tiles * S : tiles, WAVES * 64, 0, st>>>(
+      p, S, split ? static_cast<int*>(ws.ptr) : nullptr,
+      split ? reinterpret_cast<uint64_t*>(static_cast<char*>(ws.ptr) + W8_CNT_BYTES) : nullptr);
+}
+// Without a workspace the slices run in turn, in blocks small enough for the chip (the block's
+// shape does not change an output's sum, the slices do). 5 to 16 rows: one 16 x 16 block a
+// workgroup, chunks loaded one ahead, or two where slices give the waves unequal counts (16 x
+// 4096 x 4096 12.8 us against 13.9, 5 x 768 x 3072 9.3 against 10.2; f32 MFMA on the unsplit rows
+// 15.4 and 8.5). More rows: 32 x 32, or 32 x 64 in place of more than one round of those (128 x 3000
+// x 1520 13.1 us, 19.7 as 32 x 32; 64 x 4096 x 4096, one round, 24.3 against 28.9).
 template <int FM, int FN, int PF>
 static void launch_w8a32_ksplit(const W8P& p, const W8Ws& ws, hipStream_t st) {
-  const int tiles = ((p.M + 16 * FM - 1) / (16 * FM)) * ((p.N + 16 * FN - 1) / (16 * FN));
-  const int KT = (p.K + 63) / 64;
-  int S = std::max(1, std::min(256 / tiles, KT / W8_WAVES));
-  const int per = std::max(1, (KT + S - 1) / S);  // K = 0 has one empty slice
-  S = (KT + per - 1) / per;  // no empty slice
-  if ((size_t)tiles * S * FM * FN * 1024 > W8_WS_BYTES - W8_CNT_BYTES || tiles * 4 > (int)W8_CNT_BYTES) S = 1;
-  const bool split = S > 1 && ws.ptr && ws.bytes >= W8_WS_BYTES;
-  int* cnt = split ? static_cast<int*>(ws.ptr) : nullptr;
-  uint64_t* part = split ? reinterpret_cast<uint64_t*>(static_cast<char*>(ws.ptr) + W8_CNT_BYTES) : nullptr;
-  w8a32_ksplit_kernel<FM, FN, PF><<<tiles * (split ? S : 1), W8_WAVES * 64, 0, st>>>(p, S, cnt, part);
+  const int S = w8a32_slices(p, FM, FN);
+  if (S == 1 || (ws.ptr && ws.bytes >= W8_WS_BYTES)) return launch_w8a32_blocks<FM, FN, PF>(p, S, ws, st);
+  const int KT = (p.K + 63) / 64, per = (KT + S - 1) / S;
+  if (FM == 1 && per % W8_WAVES == 0) launch_w8a32_blocks<1, 1, 1, true>(p, S, ws, st);
+  else if (FM == 1) launch_w8a32_blocks<1, 1, 2, true>(p, S, ws, st);
+  else if (((p.M + 31) / 32) * ((p.N + 31) / 32) > 256) launch_w8a32_blocks<2, 4, 2, true>(p, S, ws, st);
+  else launch_w8a32_blocks<2, 2, 2, true>(p, S, ws, st);
 }
 
 template <int FM, int FN, int WAVES>

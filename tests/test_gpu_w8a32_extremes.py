@@ -156,3 +156,19 @@ def test_tiny_values(M, N, K, scale):
     # and as a whole as close as ordinary values come (about 4e-7): the lost bits are 2^-17 of 2^-118
     assert float(err.norm() / want.norm()) < 2e-6
     assert torch.equal(y[rows == 0], plain[rows == 0]) and not bool(y[rows == 2].any())
+
+
+# more slices than meet at a time (8 of a 16 x 16 block, 2 of the larger), unequal and short last ones
+@pytest.mark.parametrize("M,N,K", [(16, 40, 8208), (5, 300, 8240), (3, 100, 16384), (12, 700, 4112), (33, 200, 8208),
+                                   (20, 64, 12304), (128, 3000, 1520), (64, 1000, 4176), (200, 1024, 2064)])
+def test_slices_in_turn(M, N, K):
+    """Without a workspace the slices of K run in turn in other blocks: the same bits."""
+    print(f"w8a32 in turn M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device="cuda")
+    w8 = I.pack_linear_weight(torch.randn(N, K, generator=g, device="cuda"), weight_only=True)
+    b = torch.randn(N, generator=g, device="cuda")
+    out = torch.empty(M, N, device="cuda")
+    check(lib().bq_linear_w8a32(x.data_ptr(), w8.q.data_ptr(), M, N, K, w8.s.data_ptr(), b.data_ptr(), None, 0,
+                                out.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(out, I.linear_w8a32(x, w8, b))
