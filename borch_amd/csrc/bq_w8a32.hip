@@ -898,31 +898,43 @@ static int w8a32_common(const char* what, const float* x, const int8_t* W, int64
   }
   const uintptr_t ptrs = (uintptr_t)sW | (uintptr_t)bias | (uintptr_t)res | (uintptr_t)out;
   W8P p{x, W, (int)M, (int)N, (int)K, sW, bias, res, act, out, N % 4 == 0 && (ptrs & 15) == 0};
-  // The K-split kernel up to 511 tiles of 32 x 128 (2 a CU; 512 x 4096 x 4096 is 76 us there
-  // and 67 in the tiled one, 1024^3 15 and 22), its tile the largest that with its slices still
-  // gives the chip's CUs a workgroup each: 16 x 64 for 16 rows of 4096 x 4096 (16 x 32 12.8 us
-  // against 11.6) but 16 x 32 at 2048 x 2048 (16 x 64 8.1 us against 7.4); 32 x 128 from 160
-  // workgroups on (200 x 3072 x 768, 168 workgroups: 12.8 us, 17.5 in 336 of 32 x 64). Few rows
-  // of a short K stay with the f32 MFMA, which needs no split of x and no exchange (12 x 3000 x
-  // 1520 6.4 us against 7.6; at 16 x 2048 x 2048 8.5 against 7.4). Tiled: 128 x 128 workgroups
-  // where they fill the chip evenly (2048^3 55 us against 59 in 64 x 128), else 64 x 128
-  // (6304 x 768 x 3072, 300 tiles of 128 x 128: 108 us against 122).
+  // The K-split kernel up to 256 tiles of 32 x 128, its tile the largest that with its slices still
+  // gives the chip's CUs a workgroup each: 16 x 64 for 16 rows of 4096 x 4096 (16 x 32 12.0 us
+  // against 11.1) but 16 x 32 at 2048 x 2048 (16 x 64 8.1 us against 7.5); 32 x 128 from 160
+  // workgroups on (256 x 3072 x 768, 192 workgroups: 12.2 us, 17.0 in 384 of 32 x 64), and 32 x 64
+  // rather than 32 x 32 in more than one round of workgroups (1024 x 300 x 512: 7.0 us against
+  // 10.1), as 32 x 128 rather than 32 x 64 (951 x 640 x 640: 11.2 against 16.3). Over a K of at most
+  // five chunks 16 x 64 by four waves, whose exchange is half as long, in one round (three a CU):
+  // 256 x 3072 x 208 6.4 us, 7.2 as 32 x 128; at 384 9.7 against 9.0, and 449 x 1784 x 256, 812
+  // workgroups, 9.1 against 7.3.
+  // 5 to 12 rows of up to 2048 values, and 13 to 16 in fewer than three slices, stay with the f32
+  // MFMA, which needs no split of x and no exchange (12 x 3000 x 1520 5.8 us against 7.3, 16 x 4096 x
+  // 1280 6.6 against 7.5; 16 x 300 x 1792, three slices, 7.5 against 6.4).
+  // Tiled above 256: 64 x 64 workgroups up to 511 (1024 x 1400 x 1024 21.4 us, 27.5 K-split, 22.1 in 64
+  // x 128; 4096 x 300 x 320 10.7, 14.5 and 12.0), up to 1023 under K = 512 (2000 x 1200 x 400 15.8
+  // against 19.0; 4096 x 768 x 640 24.0 against 23.6), then 128 x 128 where they fill the chip evenly
+  // (2048^3 55 us against 59 in 64 x 128), else 64 x 128 (6304 x 768 x 3072, 300 tiles of 128 x 128:
+  // 108 us against 122).
   const auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   // workgroups a K-split tile shape can fill: its tiles times the slices of at least a chunk a wave
   const auto fill = [&](int fm, int fn) { return tiles(16 * fm, 16 * fn) * std::max<int64_t>(1, (K + 63) / 64 / W8_WAVES); };
   if (M <= WA_MMAX) {
-    if (K <= 1024 || (K <= 2048 && M <= 12)) {
+    const int fn = fill(1, 4) >= 256 ? 4 : fill(1, 2) >= 256 ? 2 : 1;
+    if (K <= 1024 || (K <= 2048 && (M <= 12 || w8a32_slices(p, 1, fn) < 3))) {
       const unsigned grid = (unsigned)((N + WM_ROWS - 1) / WM_ROWS);
       gemv_w8a32_mfma_kernel<4><<<grid, WA_WAVES * 64, 0, st>>>(x, W, (int)M, (int)N, (int)K, sW, bias, res, act, out);
       return check_launch(what);
     }
-    if (fill(1, 4) >= 256) launch_w8a32_ksplit<1, 4, 2>(p, ws, st);
-    else if (fill(1, 2) >= 256) launch_w8a32_ksplit<1, 2, 4>(p, ws, st);
+    if (fn == 4) launch_w8a32_ksplit<1, 4, 2>(p, ws, st);
+    else if (fn == 2) launch_w8a32_ksplit<1, 2, 4>(p, ws, st);
     else launch_w8a32_ksplit<1, 1, 4>(p, ws, st);
-  } else if (tiles(32, 128) < 512) {
-    if (M > 32 && fill(2, 8) >= 160) launch_w8a32_ksplit<2, 8, 1>(p, ws, st);
-    else if (fill(2, 4) >= 256) launch_w8a32_ksplit<2, 4, 2>(p, ws, st);
+  } else if (tiles(32, 128) <= 256) {
+    if (K <= 320 && tiles(16, 64) <= 768) launch_w8a32_blocks<1, 4, 1, false, 4>(p, 1, ws, st);
+    else if (M > 32 && (fill(2, 8) >= 160 || tiles(32, 64) > 256)) launch_w8a32_ksplit<2, 8, 1>(p, ws, st);
+    else if (fill(2, 4) >= 256 || tiles(32, 32) > 256) launch_w8a32_ksplit<2, 4, 2>(p, ws, st);
     else launch_w8a32_ksplit<2, 2, 2>(p, ws, st);
+  } else if (tiles(32, 128) < (K < 512 ? 1024 : 512)) {
+    launch_w8a32_tile<1, 4, 4>(p, st);
   } else {
     const int64_t t = tiles(128, 128);
     if (t >= 512 || (t >= 192 && t <= 256)) launch_w8a32_tile<1, 8, 8>(p, st);
