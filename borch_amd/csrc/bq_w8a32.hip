@@ -306,7 +306,6 @@ struct W8P {
   const float* res;  // [M, N] or null
   int act;
   float* out;        // [M, N]
-  int vec;           // N % 4 == 0 and every pointer 16-byte aligned: whole float4s
 };
 
 // Outputs of one row that a wave takes again over the effective weights f32(q) * s: lane l's
@@ -371,6 +370,8 @@ __device__ __attribute__((noinline)) W8Again w8_again(const float* x, const int8
   return W8Again{y, row};
 }
 
+typedef float v4f_u __attribute__((ext_vector_type(4), aligned(4)));
+
 // Outputs n .. n + 3 of row m from their sums; the whole wave calls it. An output whose scaled
 // sum is not finite is taken again over the effective weights f32(q) * s: the split leaves NaN
 // where x is infinite or rounds to a bf16 infinity, the sum of x * q can overflow where that of
@@ -383,11 +384,12 @@ __device__ __forceinline__ void w8_store4(const W8P& p, int m, int n, v4f v, int
   const bool in = m < p.M && n < p.N;
   const size_t o = (size_t)m * p.N + n;
   v4f s = {0.f, 0.f, 0.f, 0.f}, bias = s, res = s;  // loaded together, before the test that needs the scales
+  const bool whole = n + 3 < p.N;  // 16-byte accesses, which need 4-byte alignment only
   if (in) {
-    if (p.vec) {
-      s = *reinterpret_cast<const v4f*>(p.sW + n);
-      if (p.bias) bias = *reinterpret_cast<const v4f*>(p.bias + n);
-      if (p.res) res = *reinterpret_cast<const v4f*>(p.res + o);
+    if (whole) {
+      s = *reinterpret_cast<const v4f_u*>(p.sW + n);
+      if (p.bias) bias = *reinterpret_cast<const v4f_u*>(p.bias + n);
+      if (p.res) res = *reinterpret_cast<const v4f_u*>(p.res + o);
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -418,8 +420,8 @@ __device__ __forceinline__ void w8_store4(const W8P& p, int m, int n, v4f v, int
     if (p.res) v[e] = __fadd_rn(v[e], res[e]);
     v[e] = activate(v[e], p.act);
   }
-  if (p.vec) {
-    *reinterpret_cast<v4f*>(p.out + o) = v;
+  if (whole) {
+    *reinterpret_cast<v4f_u*>(p.out + o) = v;
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -896,8 +898,7 @@ static int w8a32_common(const char* what, const float* x, const int8_t* W, int64
     launch_gemv_w8a32(x, W, (int)M, (int)N, (int)K, sW, bias, res, act, out, st);
     return check_launch(what);
   }
-  const uintptr_t ptrs = (uintptr_t)sW | (uintptr_t)bias | (uintptr_t)res | (uintptr_t)out;
-  W8P p{x, W, (int)M, (int)N, (int)K, sW, bias, res, act, out, N % 4 == 0 && (ptrs & 15) == 0};
+  const W8P p{x, W, (int)M, (int)N, (int)K, sW, bias, res, act, out};
   // The K-split kernel up to 256 tiles of 32 x 128, its tile the largest that with its slices still
   // gives the chip's CUs a workgroup each: 16 x 64 for 16 rows of 4096 x 4096 (16 x 32 12.0 us
   // against 11.1) but 16 x 32 at 2048 x 2048 (16 x 64 8.1 us against 7.5); 32 x 128 from 160
