@@ -570,14 +570,13 @@ def test_dwconv(dev, N, C, H, k, stride, pad):
                                    (8, 512, 4096), (7, 130, 2064),
                                    # the per-wave kernel's 128 KB LDS staging (M * K in (16384, 32768])
                                    (3, 130, 8192), (4, 257, 6144),
-                                   # the f32-MFMA GEMV up to 16 rows
+                                   # 16 rows: 16 x 64 K-split blocks over a long K, f32 MFMA over a short
                                    (16, 4096, 4096), (12, 70, 1040),
-                                   # the tiled bf16-MFMA kernel: 32 x 64 tiles (M <= 256), ragged
-                                   # edges, a K tail inside a 128-deep stage, K > 8192 at small M
+                                   # the K-split kernel's other blocks: ragged edges, a K tail inside a
+                                   # chunk, K > 8192 at small M
                                    (17, 300, 1040), (256, 4096, 4096), (100, 33, 2064), (5, 130, 8208),
-                                   # 64 x 64 tiles (M > 256, fewer than 256 128 x 128 tiles)
                                    (300, 200, 2064), (1000, 520, 784),
-                                   # 128 x 128 tiles, and ViT-B/16's MLP shapes at b32
+                                   # 64 x 128 tiles, and ViT-B/16's MLP shapes at b32 (128 x 128, 64 x 128)
                                    (1100, 4100, 1024), (6304, 3072, 768), (6304, 768, 3072)])
 def test_w8a32_linear(dev, M, N, K):
     say(f"w8a32 M={M} N={N} K={K}")
@@ -656,7 +655,7 @@ def test_w8a32_decode_gemv_hand_cases(dev):
 @pytest.mark.parametrize("M", [3, 10, 100, 700])
 def test_w8a32_residual(dev, M):
     """The residual is added after the bias and before the activation (the W8A8 epilogue's
-    order), in every W8A32 kernel: the result equals the plain output plus the residual,
+    order), from one row to many: the result equals the plain output plus the residual,
     then ReLU, one f32 rounding each."""
     say(f"w8a32 residual M={M}")
     rng = np.random.default_rng(60 + M)

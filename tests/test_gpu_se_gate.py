@@ -1,5 +1,5 @@
-"""The squeeze-excite gates at the edges of their kernel's split: few and many channels and squeeze
-outputs, one row lane a group and several, more than one pass over channels, outputs and terms."""
+"""The squeeze-excite gates at the edges of their kernel's loops: few and many channels and squeeze
+outputs, more than one pass over channels, outputs and terms."""
 from __future__ import annotations
 
 import pytest
@@ -10,9 +10,10 @@ pytestmark = pytest.mark.gpu
 from borch_amd import int8 as I  # noqa: E402
 
 
-# one group of channels; 16 row lanes with fewer chunks and outputs than lanes, and more; 64 lanes'
-# batch edges (C = 1280 is one batch, 1284 two; 48 outputs are one, 49 two); two lanes and one at
-# C = 2048 / 2052, above them one; two passes over the groups (C = 4100); more terms than a batch
+# one group of channels; fewer chunks, channels and outputs than a batch of loads, and more (256
+# channels and four outputs a wave, eight chunks and terms); one pass of 1024 threads' channels, two
+# and the second nearly empty (1152, 1280, 2052), past four (4100); 64 outputs of the waves' first pass
+# and more (300, 9000)
 @pytest.mark.parametrize("N,C,S,HW", [(1, 4, 1, 1), (3, 12, 3, 50), (2, 32, 8, 12544), (3, 96, 4, 3136), (2, 240, 10, 784),
                                       (2, 672, 28, 196), (5, 1152, 48, 49), (2, 1280, 49, 49), (2, 1284, 48, 7),
                                       (1, 2048, 60, 49), (1, 2052, 20, 9), (1, 4100, 17, 4), (1, 64, 300, 100),

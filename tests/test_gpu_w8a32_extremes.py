@@ -30,9 +30,10 @@ def test_empty_product(M, N):
     assert torch.equal(out, torch.relu(b + r))
 
 
-# rows of the f32-MFMA kernel, the K-split one's forms and the tiled one's
-SHAPES = [(4, 64, 1024), (8, 64, 1024), (6, 300, 4096), (16, 4096, 4112), (16, 2048, 8208), (20, 768, 3072),
-          (40, 2051, 2064), (256, 3072, 1040), (600, 4099, 144), (1700, 2051, 144)]
+# rows of the GEMV, the f32-MFMA kernel, the K-split one's forms (four waves at K = 272) and the
+# tiled one's: 64 x 64, 64 x 128 and 128 x 128 workgroups, each with ragged columns and K
+SHAPES = [(4, 64, 1024), (8, 64, 1024), (6, 300, 4096), (16, 4096, 4112), (16, 2048, 8208), (20, 768, 3072), (40, 2051, 2064), (100, 300, 272),
+          (256, 3072, 1040), (700, 2051, 592), (600, 4099, 144), (1700, 2051, 144)]
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
@@ -156,6 +157,28 @@ def test_tiny_values(M, N, K, scale):
     # and as a whole as close as ordinary values come (about 4e-7): the lost bits are 2^-17 of 2^-118
     assert float(err.norm() / want.norm()) < 2e-6
     assert torch.equal(y[rows == 0], plain[rows == 0]) and not bool(y[rows == 2].any())
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES + [(17, 1, 16), (257, 2050, 320), (1030, 2055, 272), (16, 1024, 2048)])
+@pytest.mark.parametrize("act", [I.ACT_NONE, I.ACT_RELU, I.ACT_GELU])
+def test_bias_residual_and_activation(M, N, K, act):
+    """act((y + bias) + residual) of the same y, in every kernel; y within the f32 bound of float64."""
+    print(f"w8a32 epilogue M={M} N={N} K={K} act={act}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device="cuda")
+    w8 = I.pack_linear_weight(torch.randn(N, K, generator=g, device="cuda"), weight_only=True)
+    b, r = torch.randn(N, generator=g, device="cuda"), torch.randn(M, N, generator=g, device="cuda")
+    y = I.linear_w8a32(x, w8)
+    wd = (w8.q.double() * w8.s.double()[:, None]).t().contiguous()
+    want = x.double() @ wd
+    bound = (K + 3) * 2.0 ** -24 * (x.double().abs() @ wd.abs()) + 2.0 ** -23 * want.abs()
+    assert bool(((y.double() - want).abs() <= bound).all())
+    got = I.linear_w8a32(x, w8, b, act, residual=r)
+    pre = (y + b) + r
+    if act == I.ACT_GELU:
+        assert torch.allclose(got, torch.nn.functional.gelu(pre), rtol=1e-5, atol=1e-6)
+    else:
+        assert torch.equal(got, torch.relu(pre) if act == I.ACT_RELU else pre)
 
 
 # more slices than meet at a time (8 of a 16 x 16 block, 2 of the larger), unequal and short last ones

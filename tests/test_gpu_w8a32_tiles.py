@@ -22,7 +22,7 @@ def _case(M, N, K, seed=0):
 
 def _bounded(y, x, w8, b, K, act=None):
     """Within (K + 2) 2^-24 sum |x w| + 2^-24 |y| (one rounding a product and a sum, Higham's
-    gamma_K) plus the bias addition's half ulp, of the float64 result; the tiled kernels scale
+    gamma_K) plus the bias addition's half ulp, of the float64 result; the bf16 kernels scale
     the sum where the bound's weights are f32(q) * s, one more rounding of 2^-24 sum |x w|."""
     K0 = x.shape[1]
     w = w8.q.double()[:, :K0] * w8.s.double()[:, None]
@@ -33,7 +33,7 @@ def _bounded(y, x, w8, b, K, act=None):
 
 
 # rows: the f32-MFMA kernel's range and its edge, each K-split tile's remainders, the tiled
-# kernels' first problem; columns odd, below one tile and past one; K one 16-value piece, a
+# kernel's 64 x 64 and 64 x 128 workgroups; columns odd, below one tile and past one; K one 16-value piece, a
 # piece past a chunk, and slices of unequal length
 @pytest.mark.parametrize("M,N,K", [(5, 17, 16), (16, 65, 1040), (13, 129, 2064), (16, 4096, 2048), (16, 63, 8208),
                                    (6, 4100, 4096), (17, 1, 80), (31, 130, 4112), (32, 4096, 1024), (33, 127, 528),
