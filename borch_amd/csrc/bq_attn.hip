@@ -117,6 +117,22 @@ __global__ __launch_bounds__(ATT_WAVES * 64, KB <= 13 ? 4 : 2) void attention_f3
   for (int e = 0; e < 4; ++e)  // head dims 32 (e / 2) + 8 g + 4 (e % 2) .. + 3 of this lane's query
     q4[e] = q < T ? *reinterpret_cast<const float4*>(base + q * tok + 32 * (e >> 1) + 8 * g + 4 * (e & 1))
                   : make_float4(0.f, 0.f, 0.f, 0.f);
+  // v: a thread takes 4 keys x 4 head dims at a time, loaded under the softmax; up to 64 keys with
+  // k, where a workgroup is one chain of round trips (64 tokens, 3 heads 6.2 -> 6.0 us)
+  constexpr int VPER = ((KB + 1) / 2 * 128 + THREADS - 1) / THREADS;
+  float4 vr[VPER][4];
+  auto load_v = [&]() {
+#pragma unroll
+    for (int i = 0; i < VPER; ++i) {
+      const int idx = tid + i * THREADS, kq = ((idx >> 3) & 7) + 8 * (idx >> 7), c4 = (idx & 7) + 8 * ((idx >> 6) & 1);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        vr[i][e] = 4 * kq + e < T ? *reinterpret_cast<const float4*>(base + (4 * kq + e) * tok + 2 * D + 4 * c4)
+                                  : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if constexpr (KB <= 4) load_v();
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int idx = tid + i * THREADS, key = idx >> 4, c = idx & 15;
@@ -132,20 +148,6 @@ __global__ __launch_bounds__(ATT_WAVES * 64, KB <= 13 ? 4 : 2) void attention_f3
   }
   __syncthreads();
 
-  // v: a thread takes 4 keys x 4 head dims at a time
-  constexpr int VPER = ((KB + 1) / 2 * 128 + THREADS - 1) / THREADS;
-  float4 vr[VPER][4];
-  auto load_v = [&]() {
-#pragma unroll
-    for (int i = 0; i < VPER; ++i) {
-      const int idx = tid + i * THREADS, kq = ((idx >> 3) & 7) + 8 * (idx >> 7), c4 = (idx & 7) + 8 * ((idx >> 6) & 1);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        vr[i][e] = 4 * kq + e < T ? *reinterpret_cast<const float4*>(base + (4 * kq + e) * tok + 2 * D + 4 * c4)
-                                  : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
   const bool live = q0 < T;  // a wave past the last query only helps to stage
   v4f s[KB];
   float sum = 0.f;
@@ -164,7 +166,7 @@ __global__ __launch_bounds__(ATT_WAVES * 64, KB <= 13 ? 4 : 2) void attention_f3
       }
     }
   }
-  load_v();  // under the softmax
+  if constexpr (KB > 4) load_v();
   if (live) {
     // softmax over the keys of query q: exp((score - max) / sqrt(64)), keys past T at -inf, in
     // powers of two. The maximum is subtracted first, so that its own exponential is 1 whatever
