@@ -95,12 +95,13 @@ class Compiled:
 
     @torch.no_grad()
     def __call__(self, x):
-        key = (tuple(x.shape), x.dtype, x.device)
-        if self.tune and x.device.type == "cuda" and key not in self._tuned_keys:
+        device = x.device
+        key = (x.shape, x.dtype, device)
+        if self.tune and x.is_cuda and key not in self._tuned_keys:
             self._tuned_keys.add(key)
             self.tuned.append(_tune(self.model, x.chunk(self.split)[0] if self._split_ok(x) else x,
                                     cache=self.plan_cache))
-        if not self.graph or x.device.type != "cuda":
+        if not self.graph or not x.is_cuda:
             return self._run(x)
         entry = self._graphs.get(key)
         if entry is None:
@@ -122,7 +123,7 @@ class Compiled:
             self._graphs[key] = entry
         g, static_in, static_out, workspaces, replayed_on = entry
         static_in.copy_(x)
-        cur = torch._C._cuda_getCurrentRawStream(x.device.index)
+        cur = torch._C._cuda_getCurrentRawStream(device.index)
         if cur not in replayed_on:  # the workspaces go with this object, but not before its replays there have run
             replayed_on.add(cur)
             for ws in workspaces.values():

@@ -105,25 +105,31 @@ def _workspace(table: dict, device: torch.device, stream=None):
     return ws
 
 
-def _ws_args(device, shared=_SPLIT_WS):
+def _ws_args(device):
     """(pointer, bytes) of the current stream's split-K workspace (the graph's being made, else
-    ``shared``'s), or (None, 0) (unsplit)."""
-    table = shared if _OWNED.table is None else _OWNED.table
-    ws = None
-    if device.index is not None:  # one that is there already
-        ws = table.get((device.index, torch._C._cuda_getCurrentRawStream(device.index)))
-    if ws is None:
-        ws = _workspace(table, device)
-    return (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
+    the process's), or (None, 0) (unsplit)."""
+    return _table_args(_SPLIT_WS if _OWNED.table is None else _OWNED.table, device)
 
 
 def _w8a32_ws_args(device):
     """``_ws_args`` of the weight-only Linear. A capture that does not own its workspaces gets
     none (the slices in turn, the same bits): the stream's would be shared with every other
     graph captured there and with the eager calls on it."""
-    if _OWNED.table is None and torch.cuda.is_current_stream_capturing():
-        return None, 0
-    return _ws_args(device, _W8A32_WS)
+    table = _OWNED.table
+    if table is None:
+        if torch._C._cuda_isCurrentStreamCapturing():
+            return None, 0
+        table = _W8A32_WS
+    return _table_args(table, device)
+
+
+def _table_args(table: dict, device):
+    ws = None
+    if device.index is not None:  # one that is there already
+        ws = table.get((device.index, torch._C._cuda_getCurrentRawStream(device.index)))
+    if ws is None:
+        ws = _workspace(table, device)
+    return (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
 
 
 def _need(t: torch.Tensor, name: str, dtype: torch.dtype) -> None:
@@ -437,7 +443,8 @@ def linear_w8a32(x: torch.Tensor, w8: Int8Weight, bias=None, act=ACT_NONE, resid
         if tuple(residual.shape[:-1]) != tuple(lead) or residual.shape[-1] != N:
             raise RuntimeError(f"residual shape {tuple(residual.shape)} != output {(*lead, N)}")
         r = residual.reshape(M, N).float().contiguous()
-    ws = (None, 0) if M <= 4 and K <= 8192 else _w8a32_ws_args(x2.device)  # the GEMV splits nothing
+    split = M > 16 or K > 8192 or (M > 4 and K > 1024)  # fewer rows or shorter ones split nothing
+    ws = _w8a32_ws_args(x2.device) if split else (None, 0)
     check(lib().bq_linear_w8a32_ws(x2.data_ptr(), w8.q.data_ptr(), M, N, K, w8.s.data_ptr(), _ptr(b), _ptr(r), act,
                                    out.data_ptr(), *ws, _stream(x2)))
     return out.reshape(*lead, N)
