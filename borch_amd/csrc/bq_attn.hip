@@ -8,10 +8,11 @@
 //
 // One workgroup per (image, head, 128 queries), 8 waves of 16 queries. The products run on the
 // bf16 MFMA (16 times the f32 MFMA's rate): every f32 operand is the exact sum of three bf16
-// pieces (bq_bf16x3.h), and of the nine products of pieces the six of weight 2^-18 and above
-// are added into the f32 accumulator, smallest first. The three left out are below 2^-26 of
-// the product, under the f32 rounding of the sum; measured against float64 on N(0, 1) inputs
-// the output's relative error is 2.7e-7, where f32 MFMAs gave 3.3e-7.
+// pieces (bq_bf16x3.h), and of the nine products of pieces the six of weight 2^-18 and above are
+// added, the largest of each product into one f32 accumulator and the other five into a second.
+// The three left out are below 2^-26 of the product, under the f32 rounding of the sum; measured
+// against float64 on N(0, 1) inputs the output's relative error is 1.6e-7, where f32 MFMAs gave
+// 3.3e-7 (9.4e-8 and 1.9e-7 on flat softmaxes, scores of 0.01).
 //
 // k's planes are staged in LDS once, split there by the whole workgroup, and v's take their
 // place after the scores: 80 KB at 208 keys, so that two workgroups share a CU and one's loads
@@ -24,7 +25,7 @@
 // a 32-key step takes keys 32 s + 16 (e / 4) + 4 g + e % 4 as group g's eight, and row n of block
 // d is head dim 4 n + d, so that v is written to LDS and the output to memory in whole pieces.
 //
-// ViT-B/16 at 32 images (197 tokens, 12 heads): 69.5 -> 34.5 us; 256 tokens 88 -> 59 us (98 KB
+// ViT-B/16 at 32 images (197 tokens, 12 heads): 70 -> 35 us; 256 tokens 88 -> 59 us (98 KB
 // of LDS, one workgroup a CU).
 #include <math.h>
 
@@ -71,14 +72,17 @@ __device__ __attribute__((noinline)) void attention_f32_query(const float* base,
   orow[lane] = __fdiv_rn(o, sum);
 }
 
-// A fragment's products with another's, smallest pieces first, into acc.
-__device__ __forceinline__ v4f mfma6(const Split8& a, const Split8& b, v4f acc) {
-  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p3, b.p1, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p2, b.p2, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p1, b.p3, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p2, b.p1, acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p1, b.p2, acc, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p1, b.p1, acc, 0, 0, 0);
+// A fragment's products with another's: those of the first pieces into acc, the five smaller ones
+// into low, a sum of its own that is added last, so that each of acc's roundings stands for a whole
+// 32-deep product and not for a sixth of one (39 such roundings in one sum of 197 keys made the
+// error of flat softmaxes larger than f32 MFMAs', 2.1e-7 against 1.9e-7).
+__device__ __forceinline__ void mfma6(const Split8& a, const Split8& b, v4f& acc, v4f& low) {
+  low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p3, b.p1, low, 0, 0, 0);
+  low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p2, b.p2, low, 0, 0, 0);
+  low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p1, b.p3, low, 0, 0, 0);
+  low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p2, b.p1, low, 0, 0, 0);
+  low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p1, b.p2, low, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p1, b.p1, acc, 0, 0, 0);
 }
 
 template <int KB>  // key blocks of 16
@@ -157,13 +161,15 @@ __global__ __launch_bounds__(ATT_WAVES * 64, KB <= 13 ? 4 : 2) void attention_f3
 #pragma unroll
     for (int j = 0; j < KB; ++j) {
       s[j] = v4f{0.f, 0.f, 0.f, 0.f};
+      v4f low = s[j];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const unsigned char* at = kv + (16 * j + n) * 128 + (((4 * t + g) ^ ((n >> 1) & 7)) << 4);
         const Split8 kf = {*reinterpret_cast<const v8bf*>(at), *reinterpret_cast<const v8bf*>(at + PLANE),
                            *reinterpret_cast<const v8bf*>(at + 2 * PLANE)};
-        s[j] = mfma6(kf, qf[t], s[j]);
+        mfma6(kf, qf[t], s[j], low);
       }
+      s[j] += low;
     }
   }
   if constexpr (KB > 4) load_v();
@@ -226,9 +232,9 @@ __global__ __launch_bounds__(ATT_WAVES * 64, KB <= 13 ? 4 : 2) void attention_f3
 
   // O^T = v^T E^T with the unnormalised exponentials E, then O / sum (the normalisation moves past
   // the f32 sums, within their bound): block d, lane (n, g), register r -> dim 16 g + 4 r + d, query q
-  v4f o[4];
+  v4f o[4], low[4];
 #pragma unroll
-  for (int d = 0; d < 4; ++d) o[d] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int d = 0; d < 4; ++d) o[d] = low[d] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int t = 0; t < STEPS; ++t) {
     const v4f e0 = s[2 * t], e1 = s[2 * t + 1];
@@ -238,7 +244,7 @@ __global__ __launch_bounds__(ATT_WAVES * 64, KB <= 13 ? 4 : 2) void attention_f3
       const unsigned char* at = kv + t * ATT_DH * 64 + (d * 16 + n) * 64 + ((g ^ ((n >> 2) & 3)) << 4);
       const Split8 vf = {*reinterpret_cast<const v8bf*>(at), *reinterpret_cast<const v8bf*>(at + PLANE),
                          *reinterpret_cast<const v8bf*>(at + 2 * PLANE)};
-      o[d] = mfma6(vf, ef, o[d]);
+      mfma6(vf, ef, o[d], low[d]);
     }
   }
   if constexpr (KB % 2) {
@@ -251,14 +257,16 @@ __global__ __launch_bounds__(ATT_WAVES * 64, KB <= 13 ? 4 : 2) void attention_f3
       const unsigned char* at = kv + TAIL + (d * 16 + n) * 32 + g * 8;
       const v4s v1 = *reinterpret_cast<const v4s*>(at), v2 = *reinterpret_cast<const v4s*>(at + PLANE),
                 v3 = *reinterpret_cast<const v4s*>(at + 2 * PLANE);
-      o[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v3, e1, o[d], 0, 0, 0);
-      o[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v2, e2, o[d], 0, 0, 0);
-      o[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v1, e3, o[d], 0, 0, 0);
-      o[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v2, e1, o[d], 0, 0, 0);
-      o[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v1, e2, o[d], 0, 0, 0);
+      low[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v3, e1, low[d], 0, 0, 0);
+      low[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v2, e2, low[d], 0, 0, 0);
+      low[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v1, e3, low[d], 0, 0, 0);
+      low[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v2, e1, low[d], 0, 0, 0);
+      low[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v1, e2, low[d], 0, 0, 0);
       o[d] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v1, e1, o[d], 0, 0, 0);
     }
   }
+#pragma unroll
+  for (int d = 0; d < 4; ++d) o[d] += low[d];
   float* orow = out + ((size_t)b * T + q) * D + (size_t)h * ATT_DH;
   float4 y[4];
   // taken again: an output that is not finite, or (zero aside) below 2^-109, where the up to 2^-134
