@@ -25,7 +25,7 @@
 // a 32-key step takes keys 32 s + 16 (e / 4) + 4 g + e % 4 as group g's eight, and row n of block
 // d is head dim 4 n + d, so that v is written to LDS and the output to memory in whole pieces.
 //
-// ViT-B/16 at 32 images (197 tokens, 12 heads): 70 -> 35 us; 256 tokens 88 -> 59 us (98 KB
+// ViT-B/16 at 32 images (197 tokens, 12 heads): 70 -> 35 us; 256 tokens 86 -> 53 us (98 KB
 // of LDS, one workgroup a CU).
 #include <math.h>
 
